@@ -52,7 +52,8 @@ struct alignas(32) ConeRay {
 };
 
 struct ConeEnt {
-  uint32_t col;   // i * ny + j
+  uint32_t col;   // byte offset of column i * ny + j in the volume, or (volumes
+                  // of 4 GiB and more) the column index
   float alpha;
 };
 
@@ -76,6 +77,10 @@ using BpRec = uint4;
 struct ConeArgs {
   int na, nh, nv, nx, ny, nz;
   int mid;               // first detector row above the source
+  int fp_blocks;         // FP workgroups per ray
+  int fp_threads;        // their threads, one detector row each
+  int fp_tile_a;         // angles per ray tile of the FP
+  int fp_big;            // entries hold column indices instead of byte offsets
   int bp_stride;         // BP row distance of adjacent lanes
   int bp_unique;         // stride guarantees distinct slices per instruction
   int bp_main_safe;      // source inside the volume's z range
@@ -87,6 +92,7 @@ struct ConeArgs {
   float zb, zt;          // volume bottom / top relative to source z
   const float *alim;     // [nv] walk parameter where row v leaves the volume's
                          // z range (>= 2 where it never does)
+  const float *ain;      // [nv] walk parameter until which row v is a slice inside
   float pzbz, pzbz1, inv_dz;
   float pzdv, z1, znm;   // BP safe-row bounds (c2D.cpp:993-1000)
   double vx, vy, dx, dy; // volume xy origin and voxel size
@@ -135,15 +141,19 @@ __device__ inline double wave_sum64(double v) {
   return v;
 }
 
-// Partial of a 256-thread workgroup: the lanes' values summed per wavefront,
-// then the four wavefronts in order into part[idx].  Every thread of the
-// workgroup calls it (it synchronises).
-__device__ inline void block_part256(double v, double *part, size_t idx) {
+// Partial of a workgroup of at most 256 threads: the lanes' values summed
+// per wavefront, then the wavefronts in order into part[idx].  Every thread
+// of the workgroup calls it (it synchronises).
+__device__ inline void block_part(double v, double *part, size_t idx) {
   __shared__ double sh[4];
   v = wave_sum64(v);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
-  if (threadIdx.x == 0) part[idx] = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+  if (threadIdx.x == 0) {
+    double s = sh[0];
+    for (unsigned w = 1; w < blockDim.x / 64; ++w) s += sh[w];
+    part[idx] = s;
+  }
 }
 
 }  // namespace ccpi

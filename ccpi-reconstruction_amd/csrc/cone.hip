@@ -14,10 +14,11 @@
 // Mapping to CDNA4:
 //   plan     one lane per (angle, h) ray walks the xy grid in double and
 //            writes the ray's (cell, alpha) list to HBM once per geometry.
-//   FP       one workgroup per ray column and 256-row block; lanes are
-//            detector rows, so the xy walk is uniform (scalar loads of the
-//            entry list) and each segment's voxel column reads are
-//            near-contiguous in z across the wave.
+//   FP       one workgroup per ray column and block of at most 256 rows;
+//            lanes are detector rows, so the xy walk is uniform (scalar
+//            loads of the entry list) and each segment's voxel column reads
+//            are near-contiguous in z across the wave.  Workgroups of one
+//            XCD take tiles of adjacent rays and angles.
 //   BP       one wavefront per voxel column: the plan lists the column's
 //            (angle, h) rays (double footprints); the list is swept once
 //            per block of 64*S detector rows, S consecutive rows per lane,
@@ -46,6 +47,7 @@ namespace ccpi {
 template <bool FILL>
 struct WalkSink {
   ConeEnt *out;
+  uint32_t scale;   // entry per column index: the column's bytes, or 1
   int n = 0;
   // ncom bookkeeping (c2D.cpp:49-78)
   float prev = 0.f;
@@ -55,7 +57,7 @@ struct WalkSink {
 
   __device__ void emit(uint32_t col, float a) {
     if (FILL) {
-      out[n] = ConeEnt{col, a};
+      out[n] = ConeEnt{col * scale, a};
       if (n >= 1) {
         const float ai = prev * inv_dz;
         if (min_xy < 0) {
@@ -171,6 +173,7 @@ __global__ __launch_bounds__(256) void cone_walk_kernel(
   const int hlo = g.hrange[2 * a], hhi = g.hrange[2 * a + 1];
   WalkSink<FILL> sk;
   sk.out = FILL ? ents + offs[r] : nullptr;
+  sk.scale = g.fp_big ? 1u : 4u * (uint32_t)g.nz;
   sk.pzbz = g.pzbz;
   sk.inv_dz = g.inv_dz;
   sk.dz0 = g.dz[0];
@@ -294,138 +297,301 @@ struct FpRow {
   float dzv, izv;      // row's z run per unit alpha and its inverse
   float kb;            // slice base: pzbz, or pzbz + 1 for a floor-form row
   int ks;              // 1 for a floor-form row (c2D.cpp:153-167), else 0
-  int klo, khi;        // clamp of k for the boundary plane (shifted above)
-  const float *zb;     // s_vz, or s_vz + 1 above the source
   int dir4;            // byte step to the second slice: -4 below, +4 above
 };
 
-// One xy segment [a0, a1] of column `col`, ai = a0 / voxel z size: the
-// row's two slices (c2D.cpp:104-143, 153-187) weighted by their alpha
-// lengths.  Slices outside [0, nz) read 0 through the buffer range check.
-template <bool EDGE>
-__device__ inline void fp_seg(const FpRow &R, float a0, float a1, float ai,
-                              __amdgpu_buffer_rsrc_t col, float &c0, float &c1,
-                              float &w0, float &w1) {
-  int k = (int)(R.kb + ai * R.dzv);
-  if (EDGE) k -= R.ks;
-  const float az = R.zb[med3_i32(k, R.klo, R.khi)] * R.izv;
-  const float mz = min_sv(a1, az);
-  w0 = mz - a0;
-  w1 = a1 - mz;
-  const int off = k * 4;
-  c0 = buf_load_f32(col, off);
-  c1 = buf_load_f32(col, off + R.dir4);
-}
-
-__device__ inline __amdgpu_buffer_rsrc_t column_rsrc(const float *vol, uint32_t col, int nz) {
-  const uint32_t c = __builtin_amdgcn_readfirstlane(col);
-  return __builtin_amdgcn_make_buffer_rsrc((void *)(vol + (size_t)c * nz), (short)0, nz * 4,
-                                           kRsrcWord3);
-}
-
+// Segments per group of the FP.
 constexpr int kFpGroup = 8;
+// Zero entries after the last ray's (a last group reads up to kFpGroup - 1
+// of them; a read of entry ncom past an empty tail one more).
+constexpr int kFpTablePad = 2 * kFpGroup;
+// Cells of the FP's plane table below plane 0 and above plane nz.
+constexpr int kFpPad = 2;
 
-// Segments [mb, me) of one ray for the wave's rows.  Groups of kFpGroup
-// segments issue all their gathers before the in-order accumulation (the
-// sum order is the reference's).  The wave stops once the segment start
-// passes every row's exit parameter (amax_bits: a non-negative float's
-// bits, so the integer compare is the float compare).
-// Acc is the row accumulator: float (the reference's sum, c2D.cpp:104-143)
-// or double (the FP64-accumulation option: each segment's float
-// contribution is added in double).
-template <bool EDGE, class Acc>
-__device__ inline Acc fp_run(const FpRow &R, const ConeEnt *__restrict__ e,
-                             const float *__restrict__ ai, const float *vol, int nz,
-                             int mb, int me, int amax_bits, Acc acc) {
-  int m = mb;
-  for (; m + kFpGroup <= me; m += kFpGroup) {
-    if (__float_as_int(e[m - 1].alpha) >= amax_bits) return acc;
+// The entries and slice factors of one group of segments, as the scalar
+// loads deliver them (x: column byte offset or column index, y: alpha).
+typedef uint32_t fp_u16 __attribute__((ext_vector_type(16)));
+typedef uint32_t fp_u8 __attribute__((ext_vector_type(8)));
+struct FpRecs {
+  fp_u16 e;
+  fp_u8 ai;
+};
+// 4-byte aligned scalar loads: a ray's entries start anywhere in the table
+typedef fp_u16 __attribute__((aligned(4))) fp_u16a;
+typedef fp_u8 __attribute__((aligned(4))) fp_u8a;
+// A value at a uniform address of a plan table, as a scalar load.
+template <class T>
+__device__ inline T table_load(const T *p) {
+  return *(const __attribute__((address_space(4))) T *)(uintptr_t)p;
+}
+__device__ inline FpRecs fp_load(const ConeEnt *__restrict__ e, const float *__restrict__ ai) {
+  FpRecs r;
+  r.e = *(const __attribute__((address_space(4))) fp_u16a *)(uintptr_t)e;
+  r.ai = *(const __attribute__((address_space(4))) fp_u8a *)(uintptr_t)ai;
+  return r;
+}
+
+// First byte of one voxel column.  The entry holds the column's byte offset
+// when the volume's bytes fit 32 bits, its index otherwise (BIG).
+template <bool BIG>
+__device__ inline const __attribute__((address_space(1))) char *column_base(uintptr_t vol,
+                                                                            uint32_t col, int nz) {
+  return (const __attribute__((address_space(1))) char *)vol +
+         (BIG ? (size_t)col * ((size_t)nz * 4) : (size_t)col);
+}
+
+// Where a walk stands: the next segment m (its entries at e and ai) and the
+// alpha a0 at which it starts.
+struct FpPos {
+  int m;
+  float a0;
+  const ConeEnt *__restrict__ e;
+  const float *__restrict__ ai;
+};
+
+// fp_run's groups that start before alpha in_bits: every row of the wave is
+// a slice inside the volume there, so the slice needs no clamp and the reads
+// no range check (512^3 61.2 -> 60.0 ms, 256^3 4.13 -> 4.07).
+template <int DIR, bool EDGE, bool BIG, class Acc>
+__device__ inline Acc fp_inside(const FpRow &R, FpPos &P, const float *vol, int nz,
+                                uint32_t plane, int me, int in_bits, Acc acc) {
+  // one address for the three reads of a segment: the LDS address of plane
+  // k, which is the slice's byte offset in its column from a volume pointer
+  // set back by the table's own address (the floor form's -1 folded in)
+  const uint32_t base = EDGE ? plane - (uint32_t)(4 * R.ks) : plane;
+  const uintptr_t volp = (uintptr_t)vol - plane;
+  typedef const __attribute__((address_space(1))) float gfloat;
+  FpRecs r = fp_load(P.e, P.ai);
+  // the group's last segment starts at entry 6's alpha
+  while (__float_as_int(__uint_as_float(r.e[2 * kFpGroup - 3])) < in_bits) {
     float c0[kFpGroup], c1[kFpGroup], w0[kFpGroup], w1[kFpGroup];
+    uint32_t off[kFpGroup];
 #pragma unroll
     for (int j = 0; j < kFpGroup; ++j) {
-      const ConeEnt en = e[m + j];
-      fp_seg<EDGE>(R, e[m + j - 1].alpha, en.alpha, ai[m + j], column_rsrc(vol, en.col, nz),
-                   c0[j], c1[j], w0[j], w1[j]);
+      off[j] = k4_add((int)(R.kb + __uint_as_float(r.ai[j]) * R.dzv), base);
+      c0[j] = *(gfloat *)(column_base<BIG>(volp, r.e[2 * j], nz) + off[j]);
     }
+    asm volatile("" ::: "memory");   // two loads, see fp_run
+#pragma unroll
+    for (int j = 0; j < kFpGroup; ++j)
+      c1[j] = *(gfloat *)(column_base<BIG>(volp, r.e[2 * j], nz) + off[j] + 4 * DIR);
+#pragma unroll
+    for (int j = 0; j < kFpGroup; ++j) {
+      const float a1 = __uint_as_float(r.e[2 * j + 1]);
+      const float az = lds_ptr(off[j])[DIR > 0 ? 1 : 0] * R.izv;
+      const float mz = min_sv(a1, az);
+      w0[j] = mz - P.a0;
+      w1[j] = a1 - mz;
+      P.a0 = a1;
+    }
+    P.m += kFpGroup;
+    P.e += kFpGroup;
+    P.ai += kFpGroup;
+    r = fp_load(P.e, P.ai);
+    asm volatile("" ::: "memory");   // keep the load here, not at its use
 #pragma unroll
     for (int j = 0; j < kFpGroup; ++j) acc = acc + (Acc)(c0[j] * w0[j] + c1[j] * w1[j]);
-  }
-  for (; m < me; ++m) {
-    if (__float_as_int(e[m - 1].alpha) >= amax_bits) return acc;
-    const ConeEnt en = e[m];
-    float c0, c1, w0, w1;
-    fp_seg<EDGE>(R, e[m - 1].alpha, en.alpha, ai[m], column_rsrc(vol, en.col, nz), c0, c1,
-                 w0, w1);
-    acc = acc + (Acc)(c0 * w0 + c1 * w1);
+    if (P.m + kFpGroup > me) break;
   }
   return acc;
 }
 
-// One workgroup per ray and 256 detector rows, one row per lane.  Acc as
-// fp_run; with double the result is rounded once, after the d_conv scaling.
-template <class Acc>
+// Segments of one ray for the wave's rows, up to me, kFpGroup at a time: all
+// their gathers are issued before the in-order accumulation (the sum order
+// is the reference's), and the next group's entries are loaded while they
+// are in flight.  The last group may read entries past `me` (the tables are
+// padded); what lies past it is not added.  The wave stops once the segment
+// start passes every row's exit parameter (amax_bits: a non-negative
+// float's bits, so the integer compare is the float compare).
+//
+// Bound: VALU issue (12 instructions per segment and wave inside the volume,
+// 15 to 17 elsewhere; 87 % busy at 512^3) and the L1's accesses together
+// (TA 99 % busy).  The two slices of a segment are two dword loads: 64 rows
+// of one dword are near-contiguous and take about 9 L1 accesses, both in one
+// 8-byte load 15 (512^3 67.3 ms against 61.2).  One pair of wide scalar loads
+// per group replaces 16 narrow ones that each waited for the last, and the
+// column's byte offset comes from the table (20 scalar instructions per
+// segment before, 6 now).  512^3 (720 x 768^2) 80.7 -> 60.0 ms, 256^3 (360 x
+// 384^2) 4.99 -> 4.07, XTek wide cone 384^3 16.1 -> 7.6, bit-identical.
+// One xy segment [a0, a1] of a column, ai = a0 / voxel z size: the row's two
+// slices (c2D.cpp:104-143, 153-187) weighted by their alpha lengths.  Slices
+// outside [0, nz) read 0 through the buffer range check.
+// DIR: -1 / +1 every row of the wave under / over the source (the second
+// slice is one below / above the first and the boundary plane k / k + 1),
+// 0 both kinds.  EDGE: floor-form rows among them.
+// Acc is the row accumulator: float (the reference's sum, c2D.cpp:104-143)
+// or double (the FP64-accumulation option: each segment's float
+// contribution is added in double).
+template <int DIR, bool EDGE, bool BIG, class Acc>
+__device__ inline Acc fp_run(const FpRow &R, FpPos P, const float *vol, int nz, uint32_t plane,
+                             int me, int in_bits, int amax_bits, Acc acc) {
+  if constexpr (DIR != 0)
+    if (P.m + kFpGroup <= me)
+      acc = fp_inside<DIR, EDGE, BIG, Acc>(R, P, vol, nz, plane, me, in_bits, acc);
+  float c0[kFpGroup], c1[kFpGroup], w0[kFpGroup], w1[kFpGroup];
+  auto gather = [&](const FpRecs &r) {
+#pragma unroll
+    for (int j = 0; j < kFpGroup; ++j) {
+      const __amdgpu_buffer_rsrc_t col = __builtin_amdgcn_make_buffer_rsrc(
+          (void *)column_base<BIG>((uintptr_t)vol, r.e[2 * j], nz), (short)0, nz * 4, kRsrcWord3);
+      const float a1 = __uint_as_float(r.e[2 * j + 1]);
+      int k = (int)(R.kb + __uint_as_float(r.ai[j]) * R.dzv);
+      if constexpr (EDGE) k -= R.ks;
+      // outside [-1, nz] both slices are outside the volume
+      k = med3_m2s(k, nz + 1);
+      const int up = DIR == 0 ? (R.dir4 > 0 ? 4 : 0) : (DIR > 0 ? 4 : 0);
+      const float az = *lds_ptr(k4_add(k, plane) + up) * R.izv;
+      const float mz = min_sv(a1, az);
+      w0[j] = mz - P.a0;
+      w1[j] = a1 - mz;
+      const int off = k * 4;
+      c0[j] = buf_load_f32(col, off);
+      int off1 = off + (DIR == 0 ? R.dir4 : 4 * DIR);
+      if constexpr (DIR > 0) asm("" : "+v"(off1));   // two loads, see above
+      c1[j] = buf_load_f32(col, off1);
+      P.a0 = a1;
+    }
+    P.m += kFpGroup;
+    P.e += kFpGroup;
+    P.ai += kFpGroup;
+  };
+  if (P.m + kFpGroup <= me) {
+    FpRecs r = fp_load(P.e, P.ai);
+    do {
+      if (__float_as_int(P.a0) >= amax_bits) return acc;
+      gather(r);
+      r = fp_load(P.e, P.ai);
+      asm volatile("" ::: "memory");   // keep the load here, not at its use
+#pragma unroll
+      for (int j = 0; j < kFpGroup; ++j) acc = acc + (Acc)(c0[j] * w0[j] + c1[j] * w1[j]);
+    } while (P.m + kFpGroup <= me);
+  }
+  const int left = me - P.m;
+  if (left > 0 && __float_as_int(P.a0) < amax_bits) {
+    gather(fp_load(P.e, P.ai));
+#pragma unroll
+    for (int j = 0; j < kFpGroup; ++j)
+      if (j < left) acc = acc + (Acc)(c0[j] * w0[j] + c1[j] * w1[j]);
+  }
+  return acc;
+}
+
+// Ray tiles of the FP: consecutive workgroups of one XCD take a tile of
+// adjacent angles x adjacent rays, whose walks cross mostly the same columns
+// at the same time, so the columns are read from that XCD's L2.  512^3, ms
+// per FP and bytes fetched from beyond L2: rays dealt to the XCDs in turn
+// 83 / 601 GB; tiles of 16 x 16 67.7, 1 x 64 78.4, 8 x 32 72.7, 32 x 8 66.1;
+// with the loads as they are now 32 x 8 60.8, 64 x 8 60.0 / 203 GB, 128 x 8
+// 59.7, 128 x 4 60.6; 256^3 4.07 to 4.10 for all four.
+constexpr int kFpTileA = 64, kFpTileH = 8;
+
+// One workgroup per ray and block of detector rows, one row per lane.  Acc
+// as fp_run; with double the result is rounded once, after the d_conv
+// scaling.
+template <bool BIG, class Acc>
 __global__ __launch_bounds__(kFpRows) void cone_fp_kernel(
     ConeArgs g, const ConeRay *__restrict__ rays, const ConeEnt *__restrict__ ents,
     const float *__restrict__ eai, const float *__restrict__ vol, float *__restrict__ sino,
     int acc_in, double *__restrict__ norm) {
-  extern __shared__ float s_vz[];
-  for (int q = threadIdx.x; q <= g.nz; q += kFpRows) s_vz[q] = g.vz[q];
+  extern __shared__ float smem[];
+  const int nrays = g.na * g.nh;
+  // workgroup -> (row block, angle, column) through the XCD's tile
+  const int wgs = g.fp_tile_a * kFpTileH;
+  const int xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
+  const int tile = (local / wgs) * kXcds + xcd, within = local % wgs;
+  const int nth = (g.nh + kFpTileH - 1) / kFpTileH;
+  const int nta = (g.na + g.fp_tile_a - 1) / g.fp_tile_a;
+  const int rb = tile / (nth * nta), tah = tile - rb * (nth * nta);
+  const int a = (tah / nth) * g.fp_tile_a + within / kFpTileH;
+  const int h = (tah % nth) * kFpTileH + within % kFpTileH;
+  if (rb >= g.fp_blocks || a >= g.na || h >= g.nh) return;
+  const int r = a * g.nh + h;
+  // slice planes, clamped at both ends: plane q at s_vz[q + kFpPad]
+  for (int q = threadIdx.x; q < g.nz + 1 + 2 * kFpPad; q += blockDim.x)
+    smem[q] = g.vz[min(max(q - kFpPad, 0), g.nz)];
   __syncthreads();
-  // (ray, row block); grouping rays per XCD measured slower here than the
-  // hardware's round-robin spread
-  const int r = blockIdx.x;
-  const int v0 = blockIdx.y * kFpRows + threadIdx.x;
-  // lanes past the last row mirror row nv - 1 and store nothing, so the
-  // wave-wide reduction below sees every lane
-  const bool live = v0 < g.nv;
-  const int v = live ? v0 : g.nv - 1;
-  const int h = r % g.nh;
-  const ConeRay R = rays[r];
-  float *out = sino + (size_t)r * g.nv + v;
-  Acc acc = acc_in ? (Acc)*out : (Acc)0;
-  // A row whose ray has left the volume's z range at the start of a
-  // segment adds nothing from there on (c2D.cpp:153-187 break): the wave
-  // stops at the largest such walk parameter of its rows.
-  float amax = g.alim[v];
+  // the wave's first row (uniform: the walk stays in scalar registers)
+  const int wv0 =
+      __builtin_amdgcn_readfirstlane(rb * (int)blockDim.x + (int)(threadIdx.x & ~63u));
+  double ss = 0.0;
+  if (wv0 < g.nv) {
+    const int v0 = wv0 + (threadIdx.x & 63);
+    // lanes past the last row mirror row nv - 1 and store nothing, so the
+    // wave-wide reduction below sees every lane
+    const bool live = v0 < g.nv;
+    const int v = live ? v0 : g.nv - 1;
+    ConeRay R;
+    R.off = table_load(&rays[r].off);
+    R.n = table_load(&rays[r].n);
+    R.ncom = table_load(&rays[r].ncom);
+    R.min_v = table_load(&rays[r].min_v);
+    float *out = sino + (size_t)r * g.nv + v;
+    Acc acc = acc_in ? (Acc)*out : (Acc)0;
+    // A row whose ray has left the volume's z range at the start of a
+    // segment adds nothing from there on (c2D.cpp:153-187 break): the wave
+    // stops at the largest such walk parameter of its rows.
+    // Until the smallest ain of its rows all of them are a slice inside.
+    float amax = g.alim[v], ain = g.ain[v];
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d, 64));
-  const int amax_bits = __builtin_amdgcn_readfirstlane(__float_as_int(amax));
-  if (R.n > 1) {
-    const int nz = g.nz;
-    const bool lower = v < g.mid;
-    FpRow row;
-    row.dzv = g.dz[v];
-    row.izv = g.iz[v];
-    row.klo = lower ? 0 : -1;
-    row.khi = lower ? nz : nz - 1;
-    row.zb = s_vz + (lower ? 0 : 1);
-    row.dir4 = lower ? -4 : 4;
-    row.kb = g.pzbz;
-    row.ks = 0;
-    const ConeEnt *__restrict__ e = ents + R.off;
-    const float *__restrict__ ai = eai + R.off;
-    // segments before ncom: every row uses the truncating form
-    const int ncom = min(R.ncom, R.n);
-    acc = fp_run<false, Acc>(row, e, ai, vol, nz, 1, ncom, amax_bits, acc);
-    // from ncom on, rows below min_v use the floor form (c2D.cpp:153-167)
-    const bool edge = v < R.min_v;
-    row.kb = edge ? g.pzbz1 : g.pzbz;
-    row.ks = edge ? 1 : 0;
-    acc = fp_run<true, Acc>(row, e, ai, vol, nz, ncom, R.n, amax_bits, acc);
+    for (int d = 32; d >= 1; d >>= 1) {
+      amax = fmaxf(amax, __shfl_xor(amax, d, 64));
+      ain = fminf(ain, __shfl_xor(ain, d, 64));
+    }
+    const int amax_bits = __builtin_amdgcn_readfirstlane(__float_as_int(amax));
+    const int in_bits = __builtin_amdgcn_readfirstlane(__float_as_int(ain));
+    if (R.n > 1) {
+      const int nz = g.nz;
+      const bool lower = v < g.mid;
+      FpRow row;
+      row.dzv = g.dz[v];
+      row.izv = g.iz[v];
+      row.dir4 = lower ? -4 : 4;
+      row.kb = g.pzbz;
+      row.ks = 0;
+      const uint32_t plane = lds_addr(smem) + 4u * kFpPad;
+      const int wlast = min(wv0 + 63, g.nv - 1);
+      // segments before ncom: every row uses the truncating form; from
+      // ncom on, rows below min_v use the floor form (c2D.cpp:153-167)
+      const bool edge = v < R.min_v;
+      const int ncom = wv0 < R.min_v ? min(R.ncom, R.n) : R.n;
+      FpPos P{1, table_load(&ents[R.off].alpha), ents + R.off + 1, eai + R.off + 1};
+      if (wv0 >= g.mid) {
+        acc = fp_run<1, false, BIG, Acc>(row, P, vol, nz, plane, R.n, in_bits, amax_bits, acc);
+      } else if (wlast < g.mid) {
+        acc = fp_run<-1, false, BIG, Acc>(row, P, vol, nz, plane, ncom, in_bits, amax_bits, acc);
+      } else {
+        acc = fp_run<0, true, BIG, Acc>(row, P, vol, nz, plane, ncom, in_bits, amax_bits, acc);
+      }
+      if (ncom < R.n) {
+        P = FpPos{ncom, table_load(&ents[R.off + ncom - 1].alpha), ents + R.off + ncom,
+                  eai + R.off + ncom};
+        row.kb = edge ? g.pzbz1 : g.pzbz;
+        row.ks = edge ? 1 : 0;
+        if (wlast < g.mid)
+          acc = fp_run<-1, true, BIG, Acc>(row, P, vol, nz, plane, R.n, in_bits, amax_bits, acc);
+        else
+          acc = fp_run<0, true, BIG, Acc>(row, P, vol, nz, plane, R.n, in_bits, amax_bits, acc);
+      }
+    }
+    const float o = (float)(acc * (Acc)g.dconv[(size_t)h * g.nv + v]);
+    if (live) *out = o;
+    ss = live ? (double)o * (double)o : 0.0;
   }
-  const float o = (float)(acc * (Acc)g.dconv[(size_t)h * g.nv + v]);
-  if (live) *out = o;
-  if (norm) block_part256(live ? (double)o * (double)o : 0.0, norm,
-                          (size_t)blockIdx.y * gridDim.x + blockIdx.x);
+  if (norm) block_part(ss, norm, (size_t)rb * nrays + r);
 }
 
 // eai[q] = ents[q - 1].alpha / voxel z size: the slice-position factor of
 // the segment ending at entry q (the same float product the FP would form).
-__global__ void cone_ai_kernel(const ConeEnt *__restrict__ ents, uint64_t n, float inv_dz,
+// Both tables end in kFpTablePad zero entries, which the FP's last group of
+// segments may read.
+__global__ void cone_ai_kernel(ConeEnt *__restrict__ ents, uint64_t n, float inv_dz,
                                float *__restrict__ eai) {
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-  for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += stride)
-    eai[q] = q ? ents[q - 1].alpha * inv_dz : 0.0f;
+  for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n + kFpTablePad;
+       q += stride) {
+    eai[q] = q && q < n ? ents[q - 1].alpha * inv_dz : 0.0f;
+    if (q >= n) ents[q] = ConeEnt{0u, 0.0f};
+  }
 }
 
 // Counts the nonzero-weight voxel operands of cone_fp_kernel (same row
@@ -1337,6 +1503,18 @@ void cone_build_plan(ConePlan &P, hipStream_t st) {
   A.ipix = 1.0 / step;
   A.hpix0 = (sy - G.h_pix[0]) / step;
 
+  {
+    // FP: the rows of a ray in workgroups of at most kFpRows lanes, as few
+    // wavefronts as hold them, spread evenly
+    const int waves = (nv + 63) / 64, per = kFpRows / 64;
+    A.fp_blocks = (waves + per - 1) / per;
+    A.fp_threads = 64 * ((waves + A.fp_blocks - 1) / A.fp_blocks);
+    // angles per ray tile: at most kFpTileA, spread evenly over the tiles
+    const int nta = (na + kFpTileA - 1) / kFpTileA;
+    A.fp_tile_a = (na + nta - 1) / nta;
+    A.fp_big = G.n_vox() * sizeof(float) > 0xffffffffull ? 1 : 0;
+  }
+
   std::vector<float> dz(nv), iz(nv), vz(nz + 1), dconv((size_t)nh * nv);
   for (int v = 0; v < nv; v++) {
     dz[v] = (float)(G.v_pix[v] - sz);
@@ -1425,8 +1603,21 @@ void cone_build_plan(ConePlan &P, hipStream_t st) {
                                    : ((double)A.zt + kLimSlices * G.vsize[2]) / d;
       alim[v] = (float)std::min(2.0, lim);
     }
+  // Walk parameter up to which a row is a slice inside the volume, by the
+  // same margin: segments that start before it have their first slice k and
+  // the next one on the row's side in [0, nz).  Negative where the source's
+  // own height does not give that.
+  std::vector<float> ain(nv, -1.0f);
+  for (int v = 0; v < nv; v++) {
+    const double d = std::fabs((double)dz[v]) * (double)A.inv_dz, z = (double)A.pzbz;
+    if (v < A.mid ? (z > (double)nz - 0.5 || z < 1.5) : z > (double)nz - 1.5) continue;
+    const double room = v < A.mid ? z - 1.0 - kLimSlices : (double)nz - 1.0 - kLimSlices - z;
+    ain[v] = (float)std::min(2.0, room / d);
+  }
   P.alim.upload(alim, st);
   A.alim = P.alim.as<float>();
+  P.ain.upload(ain, st);
+  A.ain = P.ain.as<float>();
   P.atab.upload(atab, st);
   P.hpix.upload(G.h_pix, st);
   P.hrange.upload(hr, st);
@@ -1464,12 +1655,12 @@ void cone_build_plan(ConePlan &P, hipStream_t st) {
   }
   P.n_entries = tot;
   P.offs.upload(ho, st);
-  P.ents.alloc(std::max<uint64_t>(tot, 1) * sizeof(ConeEnt));
+  P.ents.alloc((tot + kFpTablePad) * sizeof(ConeEnt));
   hipLaunchKernelGGL(cone_walk_kernel<true>, dim3(blocks), dim3(256), 0, st, A,
                      P.offs.as<uint64_t>(), nullptr, P.rays.as<ConeRay>(),
                      P.ents.as<ConeEnt>());
   CCPI_HIP(hipGetLastError());
-  P.eai.alloc(std::max<uint64_t>(tot, 1) * sizeof(float));
+  P.eai.alloc((tot + kFpTablePad) * sizeof(float));
   hipLaunchKernelGGL(cone_ai_kernel, dim3(2048), dim3(256), 0, st, P.ents.as<ConeEnt>(),
                      (uint64_t)tot, A.inv_dz, P.eai.as<float>());
   CCPI_HIP(hipGetLastError());
@@ -1504,24 +1695,36 @@ void cone_build_plan(ConePlan &P, hipStream_t st) {
 
 size_t cone_fp_norm_parts(const ConePlan &P) {
   const ConeArgs &A = P.args;
-  return (size_t)A.na * A.nh * (size_t)((A.nv + kFpRows - 1) / kFpRows);
+  return (size_t)A.na * A.nh * (size_t)A.fp_blocks;
+}
+
+template <bool BIG, class Acc>
+static void cone_fp_launch(const ConePlan &P, const float *vol, float *sino, hipStream_t st,
+                           bool acc_in, double *norm) {
+  const ConeArgs &A = P.args;
+  // ray tiles of every row block, dealt to the XCDs in turn
+  const long long tiles = (long long)A.fp_blocks * ((A.na + A.fp_tile_a - 1) / A.fp_tile_a) *
+                          ((A.nh + kFpTileH - 1) / kFpTileH);
+  const long long blocks = (tiles + kXcds - 1) / kXcds * kXcds * (A.fp_tile_a * kFpTileH);
+  CCPI_REQUIRE(blocks < (1LL << 31), CCPI_E_LIMIT, "cone FP: too many rays");
+  const size_t lds = sizeof(float) * (size_t)(A.nz + 1 + 2 * kFpPad);
+  hipLaunchKernelGGL((cone_fp_kernel<BIG, Acc>), dim3((unsigned)blocks), dim3(A.fp_threads), lds,
+                     st, A, P.rays.as<ConeRay>(), P.ents.as<ConeEnt>(), P.eai.as<float>(), vol,
+                     sino, acc_in ? 1 : 0, norm);
+  CCPI_HIP(hipGetLastError());
 }
 
 void cone_fp(const ConePlan &P, const float *vol, float *sino, hipStream_t st, bool f64,
              bool acc_in, double *norm) {
-  const ConeArgs &A = P.args;
-  dim3 grid((unsigned)(A.na * A.nh), (unsigned)((A.nv + kFpRows - 1) / kFpRows));
-  const size_t lds = sizeof(float) * (size_t)(A.nz + 1);
-  const int ai = acc_in ? 1 : 0;
-  if (f64)
-    hipLaunchKernelGGL(cone_fp_kernel<double>, grid, dim3(kFpRows), lds, st, A,
-                       P.rays.as<ConeRay>(), P.ents.as<ConeEnt>(), P.eai.as<float>(), vol,
-                       sino, ai, norm);
+  const bool big = P.args.fp_big != 0;
+  if (f64 && big)
+    cone_fp_launch<true, double>(P, vol, sino, st, acc_in, norm);
+  else if (f64)
+    cone_fp_launch<false, double>(P, vol, sino, st, acc_in, norm);
+  else if (big)
+    cone_fp_launch<true, float>(P, vol, sino, st, acc_in, norm);
   else
-    hipLaunchKernelGGL(cone_fp_kernel<float>, grid, dim3(kFpRows), lds, st, A,
-                       P.rays.as<ConeRay>(), P.ents.as<ConeEnt>(), P.eai.as<float>(), vol,
-                       sino, ai, norm);
-  CCPI_HIP(hipGetLastError());
+    cone_fp_launch<false, float>(P, vol, sino, st, acc_in, norm);
 }
 
 void cone_nnz(const ConePlan &P, unsigned long long *count, hipStream_t st) {

@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void par_fp_kernel(ParArgs g, int lr,
                                                      double *__restrict__ norm) {
   const double ss =
       par_fp_lanes<Acc>(g, blockIdx.x, blockIdx.y, threadIdx.x, lr, vol, sino, acc_in != 0);
-  if (norm) block_part256(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
+  if (norm) block_part(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
 }
 
 template <class Acc>
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void par_bp_kernel(ParArgs g,
                                                      double *__restrict__ norm) {
   const double ss = par_bp_thread<kRows, Acc>(g, blockIdx.x, blockIdx.y, threadIdx.x, sino,
                                               vol, acc_in != 0);
-  if (norm) block_part256(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
+  if (norm) block_part(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
 }
 
 // The tiled BP as one launch: blockIdx.x = tile, y = slice chunk, z = angle
@@ -85,7 +85,7 @@ __attribute__((amdgpu_waves_per_eu(par_bp_lds_min_waves<Acc>(), 8))) void par_bp
   float *dst = groups == 1 ? vol : part + (size_t)grp * g.nx * g.ny * g.nz;
   const double ss = par_bp_tile<R, Acc>(g, blockIdx.x, blockIdx.y, a_begin, a_end, hmax, ab,
                                         groups == 1 && acc_in != 0, sino, dst, smem);
-  if (norm) block_part256(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
+  if (norm) block_part(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
 }
 
 // Workgroups of par_bp_sum_kernel (a fixed grid: its norm partials are a
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void par_bp_sum_kernel(const float *__restrict
     vol[q] = o;
     ss += (double)o * (double)o;
   }
-  if (norm) block_part256(ss, norm, blockIdx.x);
+  if (norm) block_part(ss, norm, blockIdx.x);
 }
 
 // Walk table of the plan, pass 1: the number of cells of every ray (one
