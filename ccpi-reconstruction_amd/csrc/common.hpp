@@ -141,11 +141,11 @@ __device__ inline double wave_sum64(double v) {
   return v;
 }
 
-// Partial of a workgroup of at most 256 threads: the lanes' values summed
+// Partial of a workgroup of at most 1024 threads: the lanes' values summed
 // per wavefront, then the wavefronts in order into part[idx].  Every thread
 // of the workgroup calls it (it synchronises).
 __device__ inline void block_part(double v, double *part, size_t idx) {
-  __shared__ double sh[4];
+  __shared__ double sh[16];
   v = wave_sum64(v);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();

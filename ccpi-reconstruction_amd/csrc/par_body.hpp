@@ -36,95 +36,10 @@ __device__ inline uint2 load_u2(const CCPI_GLOBAL uint2 *p) {
 }
 
 // The detector line of ray (a, h) walked through the xy grid (p2D.cpp:
-// 215-458): add(x, y, l) for every crossed cell, l its xy length.
-template <class Add>
-__device__ inline void par_walk(const ParArgs &g, int a, int h, Add &&add) {
-  const int nx = g.nx, ny = g.ny;
-  const double c = gmem(g.atab)[5 * a], s = gmem(g.atab)[5 * a + 1];
-  const double hp = gmem(g.h_pix)[h];
-  const double p2x = c * g.D - s * hp;
-  const double p2y = s * g.D + c * hp;
-  if (fabs(c) < kEps) {
-    if (fabs(s) >= kEps) {  // line parallel to y (p2D.cpp:233-260)
-      const int i = (int)floor((p2x - g.ox) / g.dx);
-      if (i >= 0 && i < nx) {
-        const float l = (float)g.dy;
-        if (s < 0.0)
-          for (int j = ny - 1; j >= 0; j--) add(i, j, l);
-        else
-          for (int j = 0; j < ny; j++) add(i, j, l);
-      }
-    }
-  } else if (fabs(s) < kEps) {  // line parallel to x (p2D.cpp:261-283)
-    const int j = (int)floor((p2y - g.oy) / g.dy);
-    if (j >= 0 && j < ny) {
-      const float l = (float)g.dx;
-      if (c < 0.0)
-        for (int i = nx - 1; i >= 0; i--) add(i, j, l);
-      else
-        for (int i = 0; i < nx; i++) add(i, j, l);
-    }
-  } else {  // general line (p2D.cpp:284-458)
-    const double ix = 1.0 / c, iy = 1.0 / s;
-    const double ax0 = (g.ox - p2x) * ix, ay0 = (g.oy - p2y) * iy;
-    const double axn = (g.ox + (double)nx * g.dx - p2x) * ix;
-    const double ayn = (g.oy + (double)ny * g.dy - p2y) * iy;
-    const double amin = fmax(fmax(fmin(ax0, axn), fmin(ay0, ayn)), -g.dconv);
-    const double amax = fmin(fmin(fmax(ax0, axn), fmax(ay0, ayn)), 0.0);
-    if (amin < amax - kEps) {
-      const int sx = c > 0.0 ? 1 : -1, sy = s > 0.0 ? 1 : -1;
-      int x, y;
-      {
-        const double xface = sx > 0 ? ax0 : axn, yface = sy > 0 ? ay0 : ayn;
-        const int xin = sx > 0 ? 0 : nx - 1, yin = sy > 0 ? 0 : ny - 1;
-        bool on_x = amin == xface, on_y = amin == yface;
-        if (sx > 0 && sy < 0) {
-          if (on_y) on_x = false;
-        } else if (!(sx < 0 && sy < 0)) {
-          if (on_x) on_y = false;
-        }
-        if (on_x) {
-          x = xin;
-          y = on_y ? yin : (int)floor((p2y + amin * s - g.oy) / g.dy);
-        } else if (on_y) {
-          y = yin;
-          x = (int)floor((p2x + amin * c - g.ox) / g.dx);
-        } else {
-          x = 0;
-          y = 0;
-        }
-        x = min(max(x, 0), nx - 1);
-        y = min(max(y, 0), ny - 1);
-      }
-      const int bxs = sx > 0, bys = sy > 0;
-      double ap = amin;
-      while (x >= 0 && x < nx && y >= 0 && y < ny) {
-        const double nxa = (g.ox + (double)(x + bxs) * g.dx - p2x) * ix;
-        const double nya = (g.oy + (double)(y + bys) * g.dy - p2y) * iy;
-        const int cx = x, cy = y;
-        double nap;
-        if (nxa < nya - kEps) {
-          nap = nxa;
-          x += sx;
-        } else if (nya < nxa - kEps) {
-          nap = nya;
-          y += sy;
-        } else {
-          nap = fmax(nxa, nya);
-          x += sx;
-          y += sy;
-        }
-        add(cx, cy, (float)(nap - ap));
-        ap = nap;
-      }
-    }
-  }
-}
-
-// The walk of par_walk, G cells at a time: emit(cid, l, n) receives the
-// next n <= G cells (column index x * ny + y and xy length; n < G only for
-// the last group) in the walk's order, so a caller can issue the group's
-// gathers before it accumulates them.
+// 215-458), G cells at a time: emit(cid, l, n) receives the next n <= G
+// cells (column index x * ny + y and xy length; n < G only for the last
+// group) in the walk's order, so a caller can issue the group's gathers
+// before it accumulates them.
 template <int G, class Emit>
 __device__ inline void par_walk_groups(const ParArgs &g, int a, int h, Emit &&emit) {
   const int nx = g.nx, ny = g.ny;
@@ -160,7 +75,7 @@ __device__ inline void par_walk_groups(const ParArgs &g, int a, int h, Emit &&em
         emit(cid, l, min(G, nx - i0));
       }
     }
-  } else {  // general line (p2D.cpp:284-458), steps as par_walk
+  } else {  // general line (p2D.cpp:284-458)
     const double ix = 1.0 / c, iy = 1.0 / s;
     const double ax0 = (g.ox - p2x) * ix, ay0 = (g.oy - p2y) * iy;
     const double axn = (g.ox + (double)nx * g.dx - p2x) * ix;
@@ -252,15 +167,138 @@ __device__ inline void par_cells(const ParArgs &g, int r, int a, int h, Emit &&e
   }
 }
 
-// Cells per group of the FP's walk (or walk-table reads): in the
-// one-row-per-slice FP the group's column reads are all in flight before
-// the in-order accumulation
+// Cells per group of the FP: in the one-row-per-slice FP the group's column
+// reads are all in flight before the accumulation.
 constexpr int kParFpGroup = 8;
 
-// FP of detector rows [v0, v0 + RC) of ray r (clipped to nv): `acc_in`
-// selects y += A x (reference f2D) or y = A x.  Returns the sum of squares
-// of the rows written.  Acc: float row sums (the reference's), or double
-// (the FP64-accumulation option; each float product added in double).
+// x of the lane that DPP control C names, within the lane's quad or half row
+// of 8 (all of them active).
+template <int C>
+__device__ inline float par_dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), C, 0xf, 0xf, true));
+}
+template <int C>
+__device__ inline double par_dpp(double x) {
+  const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)b, C, 0xf, 0xf, true);
+  const unsigned hi =
+      (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(b >> 32), C, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+constexpr int kDppMirror8 = 0x141;                           // lane i: x of 7 - i
+constexpr int kDppQuad[4] = {0x00, 0x55, 0xAA, 0xFF};        // lane i of every quad
+constexpr int kDppPair[2] = {0xA0, 0xF5};                    // lane i of every pair
+
+// acc + the products of CL adjacent lanes in lane order: x of lane 0, 1, ..
+// (all CL lanes hold the same acc and get the sum; with 8, lanes 0 .. 3 do).
+template <int CL, class Acc>
+__device__ inline Acc par_add_lanes(Acc acc, Acc x) {
+  if constexpr (CL == 1) {
+    acc = acc + x;
+  } else if constexpr (CL == 2) {
+    acc = acc + par_dpp<kDppPair[0]>(x);
+    acc = acc + par_dpp<kDppPair[1]>(x);
+  } else {
+    acc = acc + par_dpp<kDppQuad[0]>(x);
+    acc = acc + par_dpp<kDppQuad[1]>(x);
+    acc = acc + par_dpp<kDppQuad[2]>(x);
+    acc = acc + par_dpp<kDppQuad[3]>(x);
+    if constexpr (CL == 8) {
+      const Acc y = par_dpp<kDppMirror8>(x);   // lanes 0 .. 3: x of 7 .. 4
+      acc = acc + par_dpp<kDppQuad[3]>(y);
+      acc = acc + par_dpp<kDppQuad[2]>(y);
+      acc = acc + par_dpp<kDppQuad[1]>(y);
+      acc = acc + par_dpp<kDppQuad[0]>(y);
+    }
+  }
+  return acc;
+}
+
+// Rows v0 .. v0 + 3 of column cid, one row per slice (row v is slice v),
+// nval of them inside the volume; the others read as 0.
+__device__ inline float4 par_rows4(const ParArgs &g, const float *__restrict__ vol, int cid,
+                                   int v0, int nval) {
+  const CCPI_GLOBAL float *__restrict__ cv = gmem(vol) + (size_t)cid * g.nz + v0;
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (nval > 3) {
+    v = load_f4(cv);
+  } else {
+    if (nval > 0) v.x = cv[0];
+    if (nval > 1) v.y = cv[1];
+    if (nval > 2) v.z = cv[2];
+  }
+  return v;
+}
+
+// FP of detector rows v0 .. v0 + 3 of ray r from the plan's walk table (one
+// row per slice).  CL lanes share the ray's cells and the four rows: lane c
+// of them takes cells c, c + CL, .., 8 at a time, so 8 column reads are in
+// flight per lane, and the next table entries are read while they are; the
+// products are added in the walk's order (par_add_lanes), so the sums are
+// those of a lane that walks alone.  The chain of table read and gather per
+// 8 cells is what these small launches wait for (64 x 64 x 1, 90 angles
+// 0.026 -> 0.008 ms, 128 x 128 x 7, 180 angles 0.061 -> 0.035).  Returns the sum of squares
+// of the rows written (lane 0 of the CL writes).
+template <int CL, class Acc>
+__device__ inline double par_fp_table(const ParArgs &g, int r, int v0, int c,
+                                      const float *__restrict__ vol, float *__restrict__ sino,
+                                      bool acc_in) {
+  static_assert(CL == 1 || CL == 2 || CL == 4 || CL == 8, "adjacent lanes of a half row");
+  CCPI_GLOBAL float *__restrict__ out = gmem(sino) + (size_t)r * g.nv + v0;
+  const int nrow = min(4, g.nv - v0);
+  const int nval = max(0, min(nrow, g.nz - v0));
+  Acc acc[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) acc[q] = (acc_in && q < nrow) ? (Acc)out[q] : (Acc)0;
+  const unsigned long long e0 = gmem(g.woff)[r], e1 = gmem(g.woff)[r + 1];
+  uint2 ent[8];
+  auto fetch = [&](unsigned long long e) {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const unsigned long long q = e + i * CL + c;
+      ent[i] = make_uint2(0u, 0u);
+      if (q < e1) ent[i] = load_u2(gmem(g.went) + q);
+    }
+  };
+  fetch(e0);
+  for (unsigned long long e = e0; e < e1; e += 8 * CL) {
+    float4 f[8];
+    float l[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      // entries past the ray's last are column 0 with length 0: their reads
+      // are left out (a voxel that is not finite must not enter the sum)
+      const bool in = e + i * CL + c < e1;
+      l[i] = __builtin_bit_cast(float, ent[i].y);
+      f[i] = par_rows4(g, vol, (int)ent[i].x, v0, in ? nval : 0);
+    }
+    fetch(e + 8 * CL);
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      acc[0] = par_add_lanes<CL, Acc>(acc[0], (Acc)(f[i].x * l[i]));
+      acc[1] = par_add_lanes<CL, Acc>(acc[1], (Acc)(f[i].y * l[i]));
+      acc[2] = par_add_lanes<CL, Acc>(acc[2], (Acc)(f[i].z * l[i]));
+      acc[3] = par_add_lanes<CL, Acc>(acc[3], (Acc)(f[i].w * l[i]));
+    }
+  }
+  double ss = 0.0;
+  if (c == 0) {
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+      if (q < nrow) {
+        const float o = (float)acc[q];
+        out[q] = o;
+        ss += (double)o * (double)o;
+      }
+  }
+  return ss;
+}
+
+// FP of detector rows [v0, v0 + RC) of ray r (clipped to nv), the lane
+// walking the ray itself: `acc_in` selects y += A x (reference f2D) or
+// y = A x.  Returns the sum of squares of the rows written.  Acc: float row
+// sums (the reference's), or double (the FP64-accumulation option; each
+// float product added in double).
 template <int RC, class Acc = float>
 __device__ inline double par_fp_rows(const ParArgs &g, int r, int v0,
                                      const float *__restrict__ vol,
@@ -283,42 +321,25 @@ __device__ inline double par_fp_rows(const ParArgs &g, int r, int v0,
   const int nval = g.map_type == 1 ? max(0, min(nrow, nz - v0)) : 0;
   if (g.map_type == 1) {
     // kParFpGroup cells at a time: all their column reads are issued before
-    // the accumulation, which adds the cells in the walk's order (the same
-    // float operations as one cell at a time)
+    // the accumulation, which adds the cells in the walk's order
     constexpr int Q4 = RC / 4;
-    par_cells<kParFpGroup>(g, r, a, h, [&](const int *cid, const float *l, int n) {
+    par_walk_groups<kParFpGroup>(g, a, h, [&](const int *cid, const float *l, int n) {
       float4 f[kParFpGroup][Q4];
 #pragma unroll
-      for (int q = 0; q < kParFpGroup; q++) {
-        const CCPI_GLOBAL float *__restrict__ cv = gmem(vol) + (size_t)cid[q] * nz + v0;
+      for (int q = 0; q < kParFpGroup; q++)
+#pragma unroll
+        for (int q4 = 0; q4 < Q4; q4++)
+          f[q][q4] = par_rows4(g, vol, cid[q], v0 + 4 * q4, q < n ? nval - 4 * q4 : 0);
+      // cells past the group's n add 0 * l = 0
+#pragma unroll
+      for (int q = 0; q < kParFpGroup; q++)
 #pragma unroll
         for (int q4 = 0; q4 < Q4; q4++) {
-          float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-          if (q < n) {
-            if (4 * q4 + 3 < nval) {
-              v = load_f4(cv + 4 * q4);
-            } else {
-              if (4 * q4 < nval) v.x = cv[4 * q4];
-              if (4 * q4 + 1 < nval) v.y = cv[4 * q4 + 1];
-              if (4 * q4 + 2 < nval) v.z = cv[4 * q4 + 2];
-            }
-          }
-          f[q][q4] = v;
+          acc[4 * q4] = acc[4 * q4] + (Acc)(f[q][q4].x * l[q]);
+          acc[4 * q4 + 1] = acc[4 * q4 + 1] + (Acc)(f[q][q4].y * l[q]);
+          acc[4 * q4 + 2] = acc[4 * q4 + 2] + (Acc)(f[q][q4].z * l[q]);
+          acc[4 * q4 + 3] = acc[4 * q4 + 3] + (Acc)(f[q][q4].w * l[q]);
         }
-      }
-#pragma unroll
-      for (int q = 0; q < kParFpGroup; q++) {
-        if (q < n) {
-#pragma unroll
-          for (int q4 = 0; q4 < Q4; q4++) {
-            const float4 v = f[q][q4];
-            if (4 * q4 < nval) acc[4 * q4] = acc[4 * q4] + (Acc)(v.x * l[q]);
-            if (4 * q4 + 1 < nval) acc[4 * q4 + 1] = acc[4 * q4 + 1] + (Acc)(v.y * l[q]);
-            if (4 * q4 + 2 < nval) acc[4 * q4 + 2] = acc[4 * q4 + 2] + (Acc)(v.z * l[q]);
-            if (4 * q4 + 3 < nval) acc[4 * q4 + 3] = acc[4 * q4 + 3] + (Acc)(v.w * l[q]);
-          }
-        }
-      }
     });
   } else {
     par_cells<kParFpGroup>(g, r, a, h, [&](const int *cid, const float *l, int n) {
@@ -338,6 +359,266 @@ __device__ inline double par_fp_rows(const ParArgs &g, int r, int v0,
       out[q] = o;
       ss += (double)o * (double)o;
     }
+  return ss;
+}
+
+// ---- FP, the walk shared by a wavefront --------------------------------------
+//
+// The rows of a ray need the same cells, so the lanes that share a ray need
+// not all walk it.  A workgroup takes 64 adjacent rays of one angle: the
+// lanes of its first wavefront walk a ray each, 8 cells at a time, into LDS,
+// a round ahead of the others, which gather and sum the cells, lr lanes of 4
+// rows per ray and NS rays per lane.  Cells are par_walk_groups' (the same
+// steps and lengths), added in the walk's order.
+//
+// Bound: the gathers' 64 bytes per cycle and CU from L1 (TD 79 % busy, VALU
+// 62 % at 512 x 512 x 32, 360 angles).  With every lane walking, 8 lanes
+// repeated each ray's double arithmetic (35 instructions per cell against 10
+// to gather and sum it): 512 x 512 x 32 1.51 -> 0.67 ms, 383 x 383 x 29 (180
+// angles) 0.52 -> 0.23, 256 x 256 x 16 (180) 0.135 -> 0.080.  A wavefront that
+// walks for itself only (16 or 32 of its lanes) took 0.77, 0.29 and 0.121.
+
+// Walk of one ray, a step at a time (par_walk_groups' arithmetic).
+struct ParWalker {
+  double p2x, p2y, ix, iy, ap;
+  int x, y, sx, sy;    // cell and step; an axis-parallel line steps one axis
+  float l;             // its constant length, or < 0 for a general line
+  bool on;
+
+  __device__ inline void start(const ParArgs &g, int a, int h) {
+    const int nx = g.nx, ny = g.ny;
+    const double c = gmem(g.atab)[5 * a], s = gmem(g.atab)[5 * a + 1];
+    const double hp = gmem(g.h_pix)[h];
+    p2x = c * g.D - s * hp;
+    p2y = s * g.D + c * hp;
+    ix = 1.0 / c;
+    iy = 1.0 / s;
+    ap = 0.0;
+    on = false;
+    l = -1.0f;
+    x = y = sx = sy = 0;
+    if (fabs(c) < kEps) {
+      if (fabs(s) >= kEps) {  // line parallel to y (p2D.cpp:233-260)
+        x = (int)floor((p2x - g.ox) / g.dx);
+        y = s < 0.0 ? ny - 1 : 0;
+        sy = s < 0.0 ? -1 : 1;
+        l = (float)g.dy;
+        on = x >= 0 && x < nx;
+      }
+    } else if (fabs(s) < kEps) {  // line parallel to x (p2D.cpp:261-283)
+      y = (int)floor((p2y - g.oy) / g.dy);
+      x = c < 0.0 ? nx - 1 : 0;
+      sx = c < 0.0 ? -1 : 1;
+      l = (float)g.dx;
+      on = y >= 0 && y < ny;
+    } else {  // general line (p2D.cpp:284-458)
+      const double ax0 = (g.ox - p2x) * ix, ay0 = (g.oy - p2y) * iy;
+      const double axn = (g.ox + (double)nx * g.dx - p2x) * ix;
+      const double ayn = (g.oy + (double)ny * g.dy - p2y) * iy;
+      const double amin = fmax(fmax(fmin(ax0, axn), fmin(ay0, ayn)), -g.dconv);
+      const double amax = fmin(fmin(fmax(ax0, axn), fmax(ay0, ayn)), 0.0);
+      if (amin < amax - kEps) {
+        sx = c > 0.0 ? 1 : -1;
+        sy = s > 0.0 ? 1 : -1;
+        const double xface = sx > 0 ? ax0 : axn, yface = sy > 0 ? ay0 : ayn;
+        const int xin = sx > 0 ? 0 : nx - 1, yin = sy > 0 ? 0 : ny - 1;
+        bool on_x = amin == xface, on_y = amin == yface;
+        if (sx > 0 && sy < 0) {
+          if (on_y) on_x = false;
+        } else if (!(sx < 0 && sy < 0)) {
+          if (on_x) on_y = false;
+        }
+        if (on_x) {
+          x = xin;
+          y = on_y ? yin : (int)floor((p2y + amin * s - g.oy) / g.dy);
+        } else if (on_y) {
+          y = yin;
+          x = (int)floor((p2x + amin * c - g.ox) / g.dx);
+        }
+        x = min(max(x, 0), nx - 1);
+        y = min(max(y, 0), ny - 1);
+        ap = amin;
+        on = true;
+      }
+    }
+  }
+  // The next cell: its column index and length, or a column of -1 past the
+  // walk's end.
+  __device__ inline int step(const ParArgs &g, float &len) {
+    on = on && (unsigned)x < (unsigned)g.nx && (unsigned)y < (unsigned)g.ny;
+    len = 0.0f;
+    if (!on) return -1;
+    const int cid = x * g.ny + y;
+    if (l >= 0.0f) {
+      len = l;
+      x += sx;
+      y += sy;
+      return cid;
+    }
+    const double nxa = (g.ox + (double)(x + (sx > 0 ? 1 : 0)) * g.dx - p2x) * ix;
+    const double nya = (g.oy + (double)(y + (sy > 0 ? 1 : 0)) * g.dy - p2y) * iy;
+    const bool go_x = nxa < nya - kEps, go_y = nya < nxa - kEps;
+    const double nap = go_x ? nxa : (go_y ? nya : fmax(nxa, nya));
+    x += go_y ? 0 : sx;
+    y += go_x ? 0 : sy;
+    len = (float)(nap - ap);
+    ap = nap;
+    return cid;
+  }
+};
+
+// Volumes of the shared walk: their byte offsets, and the one an ended walk
+// asks for, stay below 2^32.
+constexpr size_t kParShareBytes = 0xe0000000;
+
+// Adjacent angles that one XCD's consecutive workgroups take (16 / 32 / 64:
+// 512 x 512 x 32, 360 angles 0.739 / 0.720 / 0.720 ms, 383 x 383 x 29, 180
+// angles 0.263 / 0.262 / 0.276).
+constexpr int kParTileA = 32;
+
+// Workgroup `id` -> its rays and rows: ids go to the 8 XCDs in turn, each
+// XCD's in tiles of kParTileA angles of the same 64 columns; row blocks
+// slowest.  index: the workgroup's place among the live ones.
+struct ParShareItem {
+  int a, h0, v0;
+  bool live;
+  size_t index;
+};
+__host__ __device__ inline long long par_share_items(const ParArgs &g, int lr) {
+  const long long nb = (g.nh + 63) / 64, nta = (g.na + kParTileA - 1) / kParTileA;
+  const long long tiles = (long long)((g.nv + 4 * lr - 1) / (4 * lr)) * nta * nb;
+  return (tiles + 7) / 8 * 8 * kParTileA;
+}
+__host__ __device__ inline size_t par_share_parts(const ParArgs &g, int lr) {
+  return (size_t)((g.nv + 4 * lr - 1) / (4 * lr)) * g.na * ((g.nh + 63) / 64);
+}
+__device__ inline ParShareItem par_share_item(const ParArgs &g, int lr, int id) {
+  const int nb = (g.nh + 63) / 64, nta = (g.na + kParTileA - 1) / kParTileA;
+  const int local = id >> 3;
+  const int tile = (local / kParTileA) * 8 + (id & 7);
+  const int rb = tile / (nb * nta), tab = tile - rb * (nb * nta);
+  ParShareItem it;
+  // uniform: the rays' and rows' addresses stay in scalar registers
+  it.a = __builtin_amdgcn_readfirstlane((tab / nb) * kParTileA + local % kParTileA);
+  it.h0 = __builtin_amdgcn_readfirstlane((tab % nb) * 64);
+  it.v0 = __builtin_amdgcn_readfirstlane(rb * 4 * lr);
+  it.live = it.a < g.na && it.v0 < g.nv;
+  it.index = ((size_t)rb * g.na + it.a) * nb + tab % nb;
+  return it;
+}
+
+// LDS of a workgroup of par_fp_shared: two rounds of 8 cells of 64 rays.
+struct ParShare {
+  uint2 ent[2][8][64];   // byte offset of the cell's column, float bits of its length
+  int more[2];           // the round holds cells
+};
+
+// Rows [v0, v0 + 4 lr) of rays h0 .. h0 + 63 of angle a, by a workgroup of
+// 1 + lr / NS wavefronts.  One row per slice, volumes below kParShareBytes
+// (32-bit byte offsets; the reads past the volume that a walk's end asks for
+// return 0).  VEC: nz >= 4, a lane's 4 slices in one 16-byte read that ends
+// inside the column; otherwise single reads.  Every thread of the workgroup
+// calls it (it synchronises).  Returns the thread's sum of squares of the
+// rows it wrote.
+template <int NS, bool VEC, class Acc>
+__device__ inline double par_fp_shared(const ParArgs &g, int a, int h0, int v0, int lr,
+                                       const float *__restrict__ vol,
+                                       float *__restrict__ sino, bool acc_in, ParShare &sh) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t bytes = 4u * (uint32_t)g.nz;
+  if (wave == 0) {
+    ParWalker W;
+    W.on = false;
+    if (h0 + lane < g.nh) W.start(g, a, h0 + lane);
+    for (int buf = 0;; buf ^= 1) {
+      bool more = false;
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        float len;
+        const int cid = W.step(g, len);
+        more |= cid >= 0;
+        // an ended walk's cells read past the volume (0) with length 0
+        sh.ent[buf][q][lane] =
+            make_uint2(cid >= 0 ? bytes * (uint32_t)cid : 0xf0000000u, __float_as_uint(len));
+      }
+      const bool any = __ballot(more) != 0;
+      if (lane == 0) sh.more[buf] = any ? 1 : 0;
+      __syncthreads();
+      if (!any) break;
+    }
+    return 0.0;
+  }
+  const int per = 64 / lr;              // rays of one wavefront at a time
+  const int ray0 = (wave - 1) * NS * per;
+  const int rl = lane & (lr - 1), rr = lane / lr;
+  const int v = v0 + 4 * rl;            // the lane's first row
+  const int nrow = max(0, min(4, g.nv - v)), nval = max(0, min(nrow, g.nz - v));
+  // its slices vs .. vs + 3 all exist (VEC); rows v .. take those from `off` on
+  const int vs = VEC ? min(v, g.nz - 4) : v;
+  const int off = v - vs;
+  const uint32_t voff = 4u * (uint32_t)vs;
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)vol, (short)0, (int)(bytes * (uint32_t)(g.nx * g.ny)), 0x00020000);
+  // acc[s][q + off] is row v + q of the s-th ray
+  Acc acc[NS][4];
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    const int h = h0 + ray0 + s * per + rr;
+    const CCPI_GLOBAL float *in = gmem(sino) + ((size_t)a * g.nh + h) * g.nv + v;
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+      acc[s][k] = (acc_in && h < g.nh && k >= off && k - off < nrow) ? (Acc)in[k - off] : (Acc)0;
+  }
+  for (int buf = 0;; buf ^= 1) {
+    __syncthreads();
+    if (!__builtin_amdgcn_readfirstlane(sh.more[buf])) break;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      float f[8][4], l[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const uint2 e = sh.ent[buf][q][ray0 + s * per + rr];
+        l[q] = __uint_as_float(e.y);
+        const int at = (int)(e.x + voff);
+        if constexpr (VEC) {
+          typedef unsigned u4 __attribute__((ext_vector_type(4)));
+          const u4 t = __builtin_amdgcn_raw_buffer_load_b128(rv, at, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; k++) f[q][k] = __uint_as_float(t[k]);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            f[q][k] = k < 3 ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                                  rv, k < nval ? at + 4 * k : (int)0xf0000000u, 0, 0))
+                            : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) acc[s][k] = acc[s][k] + (Acc)(f[q][k] * l[q]);
+    }
+  }
+  double ss = 0.0;
+#pragma unroll
+  for (int s = 0; s < NS; s++) {
+    const int h = h0 + ray0 + s * per + rr;
+    if (h < g.nh) {
+      CCPI_GLOBAL float *out = gmem(sino) + ((size_t)a * g.nh + h) * g.nv + v;
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (q < nrow) {
+          // a row without a slice keeps what it holds
+          float o = (acc_in && q >= nval) ? out[q] : 0.0f;
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            if (q + off == k && q < nval) o = (float)acc[s][k];
+          out[q] = o;
+          ss += (double)o * (double)o;
+        }
+    }
+  }
   return ss;
 }
 
@@ -365,14 +646,6 @@ __device__ inline double par_fp_lanes(const ParArgs &g, int bx, int by, int tid,
   const int v0 = (by * lr + (tid & (lr - 1))) * 4;
   if (v0 >= g.nv) return 0.0;
   return par_fp_rows<4, Acc>(g, r, v0, vol, sino, acc_in);
-}
-
-// Lanes per ray of the FP for nv detector rows: enough for the rows of one
-// ray (4 per lane), at most 16.
-inline int par_fp_lanes_per_ray(int nv) {
-  int lr = 1;
-  while (lr < 16 && 4 * lr < nv) lr *= 2;
-  return lr;
 }
 
 // Footprint of the voxel column [x0, xn] x [y0, yn] on the detector at the

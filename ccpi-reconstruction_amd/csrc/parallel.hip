@@ -12,12 +12,13 @@
 // the BP visits angles and columns in the reference's order.
 //
 // Mapping to CDNA4.  FP: `lr` lanes share one ray (lr = nv / 4 rounded up
-// to a power of two, at most 16), each lane walks the ray and keeps 4
-// consecutive detector rows in registers, so the lanes of a ray read one
-// contiguous run of each crossed column (16 bytes per lane) and a wave
-// covers 64 / lr adjacent rays of one angle.  BP: one voxel column per
-// lane, kRows slices in registers, pixel rows read once per (angle, h)
-// hit.
+// to a power of two, at most 16), each keeps 4 consecutive detector rows in
+// registers, so the lanes of a ray read one contiguous run of each crossed
+// column (16 bytes per lane) and a wave covers 64 / lr adjacent rays of one
+// angle.  The rays' cells come from a walk table of the plan (small
+// launches), from one wavefront of the workgroup that walks for the others,
+// or from the lane's own walk (par_body.hpp).  BP: one voxel column per
+// lane, kRows slices in registers, pixel rows read once per (angle, h) hit.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -49,6 +50,49 @@ __global__ __launch_bounds__(256) void par_fp_kernel(ParArgs g, int lr,
   const double ss =
       par_fp_lanes<Acc>(g, blockIdx.x, blockIdx.y, threadIdx.x, lr, vol, sino, acc_in != 0);
   if (norm) block_part(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
+}
+
+// FP from the plan's walk table: `lr` lanes of 4 rows and CL lanes over its
+// cells share a ray (par_fp_table), CL fastest.
+template <int CL, class Acc>
+__global__ __launch_bounds__(256) void par_fp_table_kernel(ParArgs g, int lr,
+                                                           const float *__restrict__ vol,
+                                                           float *__restrict__ sino, int acc_in,
+                                                           double *__restrict__ norm) {
+  const int c = threadIdx.x % CL, rl = threadIdx.x / CL;
+  const int r = blockIdx.x * (256 / (CL * lr)) + rl / lr;
+  const int v0 = (blockIdx.y * lr + (rl & (lr - 1))) * 4;
+  double ss = 0.0;
+  if (r < g.na * g.nh && v0 < g.nv)
+    ss = par_fp_table<CL, Acc>(g, r, v0, c, vol, sino, acc_in != 0);
+  if (norm) block_part(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
+}
+
+#ifndef PFP_TA
+#define PFP_TA 64
+#endif
+// Workgroups of one XCD take the same 64 columns of kParTileA adjacent angles
+// (par_share_item): their rays cross mostly the same cells at the same time,
+// so the volume's columns are read from that XCD's L2 (512 x 512 x 32, 360
+// angles: fetched from beyond L2 6.6e8 bytes of 1.6e10 gathered).
+// 7 waves per SIMD (72 VGPRs) cover the gathers' latency: 5 / 6 / 7 of them
+// 512 x 512 x 32 0.705 / 0.720 / 0.671 ms, 383 x 383 x 29 0.256 / 0.262 /
+// 0.227, 256 x 256 x 16 0.079 / 0.088 / 0.080; the FP64-accumulation instances
+// keep their registers.
+template <class Acc>
+constexpr int par_fp_min_waves() { return std::is_same<Acc, float>::value ? 7 : 1; }
+
+template <int NS, bool VEC, class Acc>
+__global__ __launch_bounds__(64 * (1 + 16 / 2))
+__attribute__((amdgpu_waves_per_eu(par_fp_min_waves<Acc>(), 8))) void par_fp_shared_kernel(
+    ParArgs g, int lr, const float *__restrict__ vol, float *__restrict__ sino, int acc_in,
+    double *__restrict__ norm) {
+  __shared__ ParShare sh;
+  const ParShareItem it = par_share_item(g, lr, blockIdx.x);
+  if (!it.live) return;
+  const double ss = par_fp_shared<NS, VEC, Acc>(g, it.a, it.h0, it.v0, lr, vol, sino,
+                                                acc_in != 0, sh);
+  if (norm) block_part(ss, norm, it.index);
 }
 
 template <class Acc>
@@ -315,11 +359,10 @@ void par_build_plan(ParPlan &P, hipStream_t st) {
   A.rlo = P.rlo.as<int>();
   A.rhi = P.rhi.as<int>();
   // walk table: every ray's cells, so the FP reads them instead of walking
-  // the grid in double each time.  Only for FPs of fewer than
-  // kParWalkTableWaves wavefronts: those leave SIMDs idle and are bound by
-  // the walk's FP64 work (256 x 256 x 16, 180 angles: 0.182 -> 0.122 ms);
-  // larger ones are bound by their gathers' latency, which the table's
-  // dependent load lengthens (the 64-problem mix: 25.5 -> 27.0 ms).
+  // the grid in double each time, with several lanes per ray and group of
+  // cells.  Only for FPs of fewer than kParWalkTableWaves wavefronts: those
+  // leave SIMDs idle and are bound by the walk's serial FP64 work (par_fp_form
+  // gives both sides' times).
   const size_t rays = (size_t)G.na * G.nh;
   if (par_walk_table_wanted(G)) {
     P.woff.alloc((rays + 1) * sizeof(unsigned long long));
@@ -351,32 +394,99 @@ void par_build_plan(ParPlan &P, hipStream_t st) {
   P.bp = par_bp_shape(G, A);
 }
 
-static dim3 par_fp_grid(const ParArgs &A, int &lr) {
-  const int rays = A.na * A.nh;
-  lr = par_fp_lanes_per_ray(A.nv);
-  const int rpb = 256 / lr;
-  return dim3((unsigned)((rays + rpb - 1) / rpb), (unsigned)((A.nv + 4 * lr - 1) / (4 * lr)));
+// How the FP of a geometry runs.
+enum class ParFpForm { kLanes, kTable, kShared };
+
+// kTable where the plan has a walk table (par_walk_table_wanted).  kShared for
+// the other launches with one row per slice and 32-bit byte offsets.  kLanes
+// for the rest.  Measured (ms, lanes - with the plan's table up to 8192 waves
+// - / table / shared; waves are par_fp_waves): 64 x 64 x 1, 90 angles (128
+// waves) 0.026 / 0.008 / -; 256 x 256 x 8, 90 (1021) 0.088 / 0.042 / 0.077;
+// 200 x 200 x 16, 120 (2122) 0.070 / 0.057 / 0.062; 160 x 160 x 32, 90 (2554)
+// 0.060 / 0.063 / 0.056; 256 x 256 x 16, 180 (4128) 0.135 / 0.110 / 0.080;
+// 512 x 512 x 1, 360 (4080) 0.99 / 0.28 / 0.26; 383 x 383 x 29, 180 0.52 / - /
+// 0.23; 512 x 512 x 32, 360 1.51 / - / 0.67.
+static ParFpForm par_fp_form(const ParArgs &A) {
+  if (A.map_type != 1) return ParFpForm::kLanes;
+  if (A.woff) return ParFpForm::kTable;
+  return sizeof(float) * (size_t)A.nx * A.ny * A.nz <= kParShareBytes ? ParFpForm::kShared
+                                                                     : ParFpForm::kLanes;
 }
 
-size_t par_fp_norm_parts(const ParPlan &P) {
-  int lr;
-  const dim3 g = par_fp_grid(P.args, lr);
-  return (size_t)g.x * g.y;
+// Lanes per ray's cells of the table form: the most, up to 8, that keep
+// the launch within kParTableWaves wavefronts (384 x 384 x 2, 180 angles:
+// 0.204 / 0.107 / 0.108 ms with 4 / 8 / 8 lanes at limits of 8192 / 16384 /
+// 32768; 200 x 200 x 16, 120 angles: 0.059 / 0.057 / 0.060 with 2 / 4 / 8).
+constexpr long long kParTableWaves = 16384;
+static int par_fp_cell_lanes(const ParArgs &A, int lr) {
+  const long long rows = (A.nv + 4 * lr - 1) / (4 * lr);
+  int cl = 8;
+  while (cl > 1 && (long long)A.na * A.nh * rows * lr * cl / 64 > kParTableWaves) cl /= 2;
+  return cl;
+}
+
+// Launch of one FP: its form, lanes per ray, lanes per ray's cells (table
+// form) or rays per lane (shared form), grid and threads.
+struct ParFpLaunch {
+  ParFpForm form;
+  int lr, n;
+  dim3 grid;
+  int threads;
+  size_t parts;   // norm partials
+};
+
+static ParFpLaunch par_fp_launch_of(const ParArgs &A) {
+  ParFpLaunch L{};
+  L.form = par_fp_form(A);
+  L.lr = par_fp_lanes_per_ray(A.nv);
+  L.threads = 256;
+  const long long rays = (long long)A.na * A.nh;
+  const unsigned rows = (unsigned)((A.nv + 4 * L.lr - 1) / (4 * L.lr));
+  if (L.form == ParFpForm::kShared) {
+    L.n = std::min(L.lr, 2);
+    L.threads = 64 * (1 + L.lr / L.n);
+    const long long items = par_share_items(A, L.lr);
+    CCPI_REQUIRE(items < (1LL << 31), CCPI_E_LIMIT, "parallel FP: too many rays");
+    L.grid = dim3((unsigned)items);
+    L.parts = par_share_parts(A, L.lr);
+    return L;
+  }
+  L.n = L.form == ParFpForm::kTable ? par_fp_cell_lanes(A, L.lr) : 1;
+  const int rpb = 256 / (L.lr * L.n);
+  L.grid = dim3((unsigned)((rays + rpb - 1) / rpb), rows);
+  L.parts = (size_t)L.grid.x * L.grid.y;
+  return L;
+}
+
+size_t par_fp_norm_parts(const ParPlan &P) { return par_fp_launch_of(P.args).parts; }
+
+template <class Acc>
+static void par_fp_run(const ParPlan &P, const float *vol, float *sino, hipStream_t st,
+                       bool acc_in, double *norm) {
+  using Kernel = void (*)(ParArgs, int, const float *, float *, int, double *);
+  const ParArgs &A = P.args;
+  const ParFpLaunch L = par_fp_launch_of(A);
+  Kernel k = par_fp_kernel<Acc>;
+  if (L.form == ParFpForm::kTable)
+    k = L.n == 8   ? par_fp_table_kernel<8, Acc>
+        : L.n == 4 ? par_fp_table_kernel<4, Acc>
+        : L.n == 2 ? par_fp_table_kernel<2, Acc>
+                   : par_fp_table_kernel<1, Acc>;
+  else if (L.form == ParFpForm::kShared)
+    k = A.nz >= 4 ? (L.n == 2 ? par_fp_shared_kernel<2, true, Acc>
+                              : par_fp_shared_kernel<1, true, Acc>)
+                  : (L.n == 2 ? par_fp_shared_kernel<2, false, Acc>
+                              : par_fp_shared_kernel<1, false, Acc>);
+  hipLaunchKernelGGL(k, L.grid, dim3(L.threads), 0, st, A, L.lr, vol, sino, acc_in ? 1 : 0, norm);
+  CCPI_HIP(hipGetLastError());
 }
 
 void par_fp(const ParPlan &P, const float *vol, float *sino, hipStream_t st, bool f64,
             bool acc_in, double *norm) {
-  const ParArgs &A = P.args;
-  int lr;
-  const dim3 grid = par_fp_grid(A, lr);
-  const int ai = acc_in ? 1 : 0;
   if (f64)
-    hipLaunchKernelGGL(par_fp_kernel<double>, grid, dim3(256), 0, st, A, lr, vol, sino, ai,
-                       norm);
+    par_fp_run<double>(P, vol, sino, st, acc_in, norm);
   else
-    hipLaunchKernelGGL(par_fp_kernel<float>, grid, dim3(256), 0, st, A, lr, vol, sino, ai,
-                       norm);
-  CCPI_HIP(hipGetLastError());
+    par_fp_run<float>(P, vol, sino, st, acc_in, norm);
 }
 
 size_t par_bp_scratch_floats(const ParPlan &P) {

@@ -9,6 +9,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstring>
 #include <memory>
 #include <mutex>
@@ -138,21 +139,41 @@ struct ParPlan {
   }
 };
 
+// Lanes per ray of the parallel FP for nv detector rows: enough for the rows
+// of one ray (4 per lane), at most 16.
+inline int par_fp_lanes_per_ray(int nv) {
+  int lr = 1;
+  while (lr < 16 && 4 * lr < nv) lr *= 2;
+  return lr;
+}
+
+// One detector row per slice, row v on slice v (map_type 1, p2D.cpp:22-61).
+inline bool par_one_row_per_slice(const Geometry &g) {
+  for (int v = 0; v < g.nv; v++)
+    if ((int)std::floor((g.v_pix[v] - g.origin[2]) / g.vsize[2]) != v) return false;
+  return true;
+}
+
 // Walk table of a parallel plan: built for FPs of fewer than
-// kParWalkTableWaves wavefronts (4 detector rows per lane) when its bound
+// kParWalkTableWaves wavefronts (4 detector rows per lane; kParWalkTableWavesN
+// where rows and slices do not go one to one, whose lanes would each walk:
+// the table's 8 bytes per cell are read in their place) when its bound
 // (8 bytes per cell, at most nx + ny cells per ray, plus the ray offsets)
 // is within kParWalkTableBytes.
 constexpr size_t kParWalkTableBytes = size_t(4) << 30;
-constexpr long long kParWalkTableWaves = 8192;
+constexpr long long kParWalkTableWaves = 2400, kParWalkTableWavesN = 8192;
 inline size_t par_walk_table_bound(const Geometry &g) {
   const size_t rays = (size_t)g.na * g.nh;
   return rays * 8 * (size_t)(g.nx + g.ny) + (rays + 1) * 8;
 }
 inline long long par_fp_waves(const Geometry &g) {
-  return (long long)g.na * g.nh * ((g.nv + 3) / 4) / 64;
+  const int lr = par_fp_lanes_per_ray(g.nv);
+  return (long long)g.na * g.nh * ((g.nv + 4 * lr - 1) / (4 * lr)) * lr / 64;
 }
 inline bool par_walk_table_wanted(const Geometry &g) {
-  return par_walk_table_bound(g) <= kParWalkTableBytes && par_fp_waves(g) < kParWalkTableWaves;
+  return par_walk_table_bound(g) <= kParWalkTableBytes &&
+         par_fp_waves(g) <
+             (par_one_row_per_slice(g) ? kParWalkTableWaves : kParWalkTableWavesN);
 }
 
 std::shared_ptr<ConePlan> cone_plan(const Geometry &g, hipStream_t st);
