@@ -94,12 +94,12 @@ __device__ inline double wave_sum_d(double v) {
 // BPK: the BP bodies a batch needs (1 tiled, 2 column-per-lane, 3 both);
 // a kernel holding both bodies is sized for the larger of their register
 // sets, so a batch of one kind gets the kernel of that body alone.
-// Waves per SIMD the registers must allow: the FP items and the tiled BP
-// items wait on their gathers and staged rows, and 6 waves each (a few
-// spills in the set-up) took the 64-problem mix from 23.7 to 25.6 CGLS
-// iterations/s (the BP alone at 5: 25.0; the FP alone at 6: 24.2).
+// Waves per SIMD the registers must allow.  The FP items wait on their
+// gathers: 6 waves took the 64-problem mix from 23.7 to 24.2 CGLS iterations
+// a second.  The tiled BP items: an iteration of the mix takes 30.4 / 28.3 /
+// 28.4 ms with them at 6 / 5 / 4 waves.
 template <int MODE, int BPK>
-constexpr int batch_min_waves() { return MODE == 0 || BPK == 1 ? 6 : 1; }
+constexpr int batch_min_waves() { return MODE == 0 ? 6 : BPK == 1 ? 5 : 1; }
 
 template <int RC, int MODE, int BPK>
 __global__ __launch_bounds__(256)
@@ -131,7 +131,7 @@ __attribute__((amdgpu_waves_per_eu(batch_min_waves<MODE, BPK>(), 8))) void batch
     }
     return;
   }
-  extern __shared__ float smem[];
+  extern __shared__ __align__(16) float smem[];
   const int total = off[L.count];
   for (int item = blockIdx.x; item < total; item += gridDim.x) {
     const int p = find_prob(off, L.count, item);
@@ -151,6 +151,7 @@ __attribute__((amdgpu_waves_per_eu(batch_min_waves<MODE, BPK>(), 8))) void batch
     }
     ss = wave_sum_d(ss);
     if (lane == 0) part[4 * item + wave] = ss;
+    __syncthreads();   // the next item's first block overwrites this one's LDS
   }
 }
 
@@ -315,7 +316,7 @@ void proj(const BatchRun &R, const Tuned &T, int mode, hipStream_t st) {
 
 // Item lists for row/slice blocks of `rc`.  A problem whose plan takes the
 // tiled BP gets tile items of rc slices, its staged span and angle groups
-// from the plan and as many angles per staged block as fit 32 KB.
+// from the plan and its angles per staged block for rc slices.
 void layout(BatchRun &R, int rc, hipStream_t st) {
   std::vector<int> off(4 * (R.count + 1), 0);
   R.bp_lds = 0;
@@ -330,11 +331,10 @@ void layout(BatchRun &R, int rc, hipStream_t st) {
     B.bp_tiled = S.tiled;
     R.bp_kinds |= S.tiled ? 1 : 2;
     if (S.tiled) {
-      const size_t per_angle = sizeof(float) * (size_t)S.hmax * rc + 2 * sizeof(int);
       B.bp_hmax = S.hmax;
       B.bp_groups = S.groups;
-      B.bp_ab = (int)std::max<size_t>(1, std::min<size_t>(8, (32 * 1024) / per_angle));
-      R.bp_lds = std::max(R.bp_lds, per_angle * B.bp_ab);
+      B.bp_ab = par_bp_block_angles(S.hmax, rc);
+      R.bp_lds = std::max(R.bp_lds, par_bp_tile_bytes(S.hmax, rc, B.bp_ab));
       B.bp_nbx = ((g.nx + 15) / 16) * ((g.ny + 15) / 16);
     } else {
       B.bp_nbx = (g.nx * g.ny + 255) / 256;

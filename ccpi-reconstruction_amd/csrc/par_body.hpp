@@ -21,12 +21,37 @@ __device__ inline CCPI_GLOBAL T *gmem(T *p) {
   return (CCPI_GLOBAL T *)p;
 }
 
+// A plan table at a uniform address: scalar loads, whatever memory the kernel
+// writes meanwhile (no kernel writes the tables it reads).
+#define CCPI_CONST __attribute__((address_space(4)))
+template <class T>
+__device__ inline const CCPI_CONST T *cmem(const T *p) {
+  return (const CCPI_CONST T *)(uintptr_t)p;
+}
+
 // 16 bytes at p (4-byte aligned) as one load.
 __device__ inline float4 load_f4(const CCPI_GLOBAL float *p) {
   float4 v;
   __builtin_memcpy(&v, p, sizeof(v));
   return v;
 }
+
+// LDS byte address of a shared-memory pointer.
+__device__ inline uint32_t lds_byte(const void *p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
+}
+// Reads of 16 / 4 bytes per lane straight into LDS: lane i's go to `lds` + 16
+// i / 4 i (lds uniform).  The compiler does not know them: lds_loads_done
+// waits for the wavefront's, and a barrier after it shows them to the others.
+__device__ inline void lds_load16(uint32_t lds, const CCPI_GLOBAL float *p) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(p) : "memory");
+}
+__device__ inline void lds_load4(uint32_t lds, const CCPI_GLOBAL float *p) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
+               :: "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(p) : "memory");
+}
+__device__ inline void lds_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // One 8-byte walk-table entry.
 __device__ inline uint2 load_u2(const CCPI_GLOBAL uint2 *p) {
@@ -699,7 +724,7 @@ __device__ inline ParFoot par_footprint(const ParArgs &g, TabPtr t, double x0, d
       else         { f.ymin = yn * c - x0 * s; f.ymax = y0 * c - xn * s; }
     }
     // clamp at 0: the floor can round to -1 when ymin ~ h_pix[0]
-    f.lo = f.ymin < gmem(g.h_pix)[0] ? 0 : max((int)floor(f.ymin * g.ihp - g.hp0), 0);
+    f.lo = f.ymin < cmem(g.h_pix)[0] ? 0 : max((int)floor(f.ymin * g.ihp - g.hp0), 0);
     f.hi = min((int)floor(f.ymax * g.ihp - g.hp0), g.nh - 1);
   }
   return f;
@@ -873,10 +898,20 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // the tile's square can reach (its corners' span plus a margin of 2) are
 // staged in LDS with the R rows of the lane's slices (hmax columns at most),
 // one coalesced copy per tile instead of each lane re-reading its columns'
-// rows; every lane then walks its own column's footprint (the reference's
-// FP64 arithmetic, par_footprint / par_weight) and reads the rows from LDS.
-// A footprint column outside the staged span (never expected; rounding
-// guard) is read from global memory.  Angles are visited in order, so with
+// rows, and with the columns' positions; every lane then weighs its own
+// column's footprint (the reference's FP64 arithmetic) on the staged rows.
+// Bound by vector issue, about 150 instructions per column and angle of
+// which 60 are the 16 slices' products and sums.  So there are two blocks of
+// LDS and the next one's reads go straight there while this one is summed
+// (one barrier a block, no register in between), spans are found 256 angles
+// at a time, tables are scalar loads, and where no footprint of the
+// wavefront has more than two columns (pixels about as wide as a voxel or
+// wider) both are weighed without a loop.  With the rows staged through
+// registers between two barriers and a loop over positions in global memory
+// it took: 512 x 512 x 32, 360 angles 1.40 ms, now 0.89; 383 x 383 x 29, 180
+// angles 0.44, now 0.31; 256 x 256 x 16, 180 angles 0.116, now 0.081;
+// 64 x 64 x 1, 90 angles 0.027, now 0.021.  32 slices per lane: 0.86 at
+// 512 x 512 x 32 but 0.38 at 383 x 383 x 29.  Angles are visited in order, so with
 // one angle group the result is bit-identical to par_bp_kernel; with G
 // groups (blockIdx.z) each group writes its partial sums of its angle range
 // to part[group] and par_bp_sum_kernel adds them in group order.
@@ -886,22 +921,28 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // over the column grid), slices [zc * R, zc * R + R), angles [a_begin,
 // a_end).  The result goes to `dst` (a volume-layout array), added to its
 // contents when acc_in.  Returns the thread's sum of squares of the values
-// it wrote (0 for threads outside the volume).  smem: par_bp_lds_bytes.
+// it wrote (0 for threads outside the volume).  smem: par_bp_tile_bytes,
+// 16-byte aligned; a caller with another item to do synchronises first.
 // FOLD (the batched kernel's tiled items; acc_in must be false): the
 // angles are split into `groups` ranges as par_bp_lds_kernel splits them,
 // each summed from zero, and the running sum of the groups is kept in
 // `dst` (each lane re-reads only its own writes), so one item gives bit for
 // bit what the grouped launch and par_bp_sum_kernel give into a zeroed
 // volume, without registers for a second set of sums.
+constexpr int kParBpSpans = 256;   // one per thread
 template <int R, class Acc, bool FOLD = false>
 __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, int a_end,
                               int hmax, int ab, bool acc_in, const float *__restrict__ sino,
                               float *__restrict__ dst_vol, float *smem, int groups = 1) {
-  static_assert(R % 4 == 0, "rows are staged 4 at a time");
-  float *s_rows = smem;                                 // [ab][hmax][R]
-  int *s_lo = reinterpret_cast<int *>(smem + (size_t)ab * hmax * R);
-  int *s_cnt = s_lo + ab;
-  const int tid = threadIdx.x;
+  static_assert(R % 4 == 0, "rows are read 4 at a time");
+  constexpr int Q4 = R / 4;
+  // two buffers of a block's rows, column positions and spans
+  float *s_rows = smem;                                                        // [2][ab][hmax][R]
+  double *s_hp = reinterpret_cast<double *>(smem + 2 * (size_t)ab * hmax * R);   // [2][ab][hmax]
+  int2 *s_cur = reinterpret_cast<int2 *>(s_hp + 2 * (size_t)ab * hmax);          // [2][ab]
+  int2 *s_span = s_cur + 2 * ab;                                               // [kParBpSpans]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntj = (g.ny + 15) >> 4;
   const int ti0 = (tile / ntj) * 16, tj0 = (tile % ntj) * 16;
   const int i = ti0 + (tid >> 4), j = tj0 + (tid & 15);
@@ -917,107 +958,184 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
     acc[q] = (!FOLD && acc_in && active && q < nk) ? (Acc)vcol[q] : (Acc)0;
   const double x0 = g.ox + (double)i * g.dx, xn = g.ox + (double)(i + 1) * g.dx;
   const double y0 = g.oy + (double)j * g.dy, yn = g.oy + (double)(j + 1) * g.dy;
-  // tile square
-  const double X0 = g.ox + (double)ti0 * g.dx, XN = g.ox + (double)min(ti0 + 16, g.nx) * g.dx;
-  const double Y0 = g.oy + (double)tj0 * g.dy, YN = g.oy + (double)min(tj0 + 16, g.ny) * g.dy;
+  const double hpix0 = cmem(g.h_pix)[0];
   // rows of the lane's slices that exist (one row per slice)
   const int nrow = max(0, min(R, min(nv, nz) - k0));
-  // rows of 16-byte aligned start (nv a multiple of 4) are staged 16 bytes
-  // at a time, others one float at a time
-  const bool aligned = (nv & 3) == 0;
-  constexpr int Q4 = R / 4;
+
+  // Detector columns that the tile's square can reach at angles sb ..
+  // sb + kParBpSpans - 1: its corners' span and 2 columns on each side (the
+  // footprints' own rounding), one angle per thread.  Every column of the
+  // tile projects inside its square, and the index floor(y * ihp - hp0) grows
+  // with y, so the footprints stay inside the span.
+  auto spans = [&](int sb) {
+    const int a = sb + tid;
+    if (a >= a_end) return;
+    const double X0 = g.ox + (double)ti0 * g.dx, XN = g.ox + (double)min(ti0 + 16, g.nx) * g.dx;
+    const double Y0 = g.oy + (double)tj0 * g.dy, YN = g.oy + (double)min(tj0 + 16, g.ny) * g.dy;
+    const CCPI_GLOBAL double *tab = gmem(g.atab) + 5 * a;
+    const double c = tab[0], s = tab[1];
+    const double p0 = Y0 * c - X0 * s, p1 = YN * c - X0 * s;
+    const double p2 = Y0 * c - XN * s, p3 = YN * c - XN * s;
+    const double tmin = fmin(fmin(p0, p1), fmin(p2, p3));
+    const double tmax = fmax(fmax(p0, p1), fmax(p2, p3));
+    const int lo = max((int)floor(tmin * g.ihp - g.hp0) - 2, 0);
+    const int hi = min((int)floor(tmax * g.ihp - g.hp0) + 2, nh - 1);
+    s_span[tid] = make_int2(lo, max(0, min(hi - lo + 1, hmax)));
+  };
+  // Starts the reads of angles [a0, a0 + n) into buffer `buf`: per wavefront
+  // one angle at a time, straight into LDS.  Rows of 16-byte aligned start go
+  // 16 bytes at a time, others one float at a time.  Rows past nrow are not
+  // read or not added in the end.
+  const bool aligned = ((nv & 3) | (int)((uintptr_t)sino & 15)) == 0;
+  const int have = nv - k0;             // rows of a ray from the first slice on
+  auto start = [&](int a0, int n, int buf, int sb) {
+    for (int t = wave; t < n; t += 4) {
+      const int2 sp = s_span[a0 + t - sb];
+      const int lo = __builtin_amdgcn_readfirstlane(sp.x);
+      const int cnt = __builtin_amdgcn_readfirstlane(sp.y);
+      const int slot = buf * ab + t;
+      if (lane == 0) s_cur[slot] = sp;
+      const uint32_t row_lds = lds_byte(s_rows + (size_t)slot * hmax * R);
+      const CCPI_GLOBAL float *p = gmem(sino) + ((size_t)(a0 + t) * nh + lo) * nv + k0;
+      if (aligned) {
+        for (int hh = 0; hh < cnt; hh += 64 / Q4) {
+          const int r = hh + lane / Q4, q = 4 * (lane % Q4);
+          if (r < cnt && q < have) lds_load16(row_lds + hh * (4 * R), p + (size_t)r * nv + q);
+        }
+      } else {
+        for (int hh = 0; hh < cnt; hh += 64 / R) {
+          const int r = hh + lane / R, q = lane % R;
+          if (r < cnt && q < have) lds_load4(row_lds + hh * (4 * R), p + (size_t)r * nv + q);
+        }
+      }
+      const uint32_t hp_lds = lds_byte(s_hp + (size_t)slot * hmax);
+      const CCPI_GLOBAL float *hp = (const CCPI_GLOBAL float *)(gmem(g.h_pix) + lo);
+      for (int e = 0; e < 2 * cnt; e += 64)
+        if (e + lane < 2 * cnt) lds_load4(hp_lds + 4 * e, hp + e + lane);
+    }
+  };
+  // angle range of group `grp` (one group: all)
   const int ngrp = FOLD ? groups : 1;
-  for (int grp = 0; grp < ngrp; grp++) {
-    const int ga = FOLD ? a_begin + (int)((long long)(a_end - a_begin) * grp / groups) : a_begin;
-    const int gb =
-        FOLD ? a_begin + (int)((long long)(a_end - a_begin) * (grp + 1) / groups) : a_end;
-    if (FOLD) {
+  auto group_begin = [&](int grp) {
+    return FOLD ? a_begin + (int)((long long)(a_end - a_begin) * grp / groups) : a_begin;
+  };
+  int grp = 0, a0 = a_begin, gb = FOLD ? group_begin(1) : a_end, buf = 0;
+  int sb = a0;
+  spans(sb);
+  __syncthreads();
+  start(a0, min(ab, gb - a0), 0, sb);
+  for (;;) {
+    const int nblk = min(ab, gb - a0);
+    const bool group_ends = a0 + ab >= gb;
+    const int next = group_ends ? gb : a0 + ab;
+    const int next_gb = group_ends && grp + 1 < ngrp ? group_begin(grp + 2) : gb;
+    // the block's reads have landed, and everybody is done with the other buffer
+    lds_loads_done();
+    __syncthreads();
+    if (next < next_gb) {
+      if (next + ab > sb + kParBpSpans) {
+        sb = next;
+        spans(sb);
+        __syncthreads();
+      }
+      start(next, min(ab, next_gb - next), buf ^ 1, sb);
+    }
+    if (active) {
+      for (int t = 0; t < nblk; t++) {
+        const CCPI_CONST double *tab = cmem(g.atab) + 5 * (a0 + t);
+        const double c = tab[0], s = tab[1];
+        const int slot = buf * ab + t;
+        const int slo = s_cur[slot].x, scnt = s_cur[slot].y;
+        const float *rows_t = s_rows + (size_t)slot * hmax * R;
+        const double *hp_t = s_hp + (size_t)slot * hmax;
+        auto add = [&](const float *pr, float wf) {
+#pragma unroll
+          for (int q4 = 0; q4 < Q4; q4++) {
+            const float4 v = *reinterpret_cast<const float4 *>(pr + 4 * q4);
+            acc[4 * q4] = acc[4 * q4] + (Acc)(v.x * wf);
+            acc[4 * q4 + 1] = acc[4 * q4 + 1] + (Acc)(v.y * wf);
+            acc[4 * q4 + 2] = acc[4 * q4 + 2] + (Acc)(v.z * wf);
+            acc[4 * q4 + 3] = acc[4 * q4 + 3] + (Acc)(v.w * wf);
+          }
+        };
+        if (!(fabs(c) < kEps || fabs(s) < kEps)) {
+          // General line: par_footprint and par_weight value for value
+          // (p2D.cpp:881-938).  The footprint's first column lies at or
+          // before ymin, so columns as wide as a voxel's shadow or wider leave
+          // at most two more; both are weighed without a loop when that
+          // holds for the whole wavefront and they are staged.
+          double ymin, ymax;
+          if (c > 0.0) {
+            if (s > 0.0) { ymin = y0 * c - xn * s; ymax = yn * c - x0 * s; }
+            else         { ymin = y0 * c - x0 * s; ymax = yn * c - xn * s; }
+          } else {
+            if (s > 0.0) { ymin = yn * c - xn * s; ymax = y0 * c - x0 * s; }
+            else         { ymin = yn * c - x0 * s; ymax = y0 * c - xn * s; }
+          }
+          const int lo = ymin < hpix0 ? 0 : max((int)floor(ymin * g.ihp - g.hp0), 0);
+          const int hi = min((int)floor(ymax * g.ihp - g.hp0), nh - 1);
+          const int hh = lo - slo;
+          const double e0 = ymin + kEps;
+          bool quick = hh >= 0 && hh + 2 < scnt && hi <= lo + 2;
+          if (quick) quick = !(hp_t[hh] > e0);
+          if (__ballot(!quick) == 0) {
+            const double t2 = tab[2], t3 = tab[3], l = tab[4];
+            const double ybot = ymin + t2, ytop = ymax - t2, e1 = ymax - kEps;
+            const float *pr = rows_t + (hh + 1) * R;
+#pragma unroll
+            for (int u = 1; u <= 2; u++) {
+              const double hp = hp_t[hh + u];
+              const bool rise = hp < ybot, flat = !rise && hp <= ytop;
+              const double d = rise ? hp - ymin : ymax - hp;
+              const double w = flat ? l : l * d * t3;
+              if (lo + u <= hi && hp > e0 && (rise || flat || hp < e1))
+                add(pr + (u - 1) * R, (float)w);
+            }
+            continue;
+          }
+        }
+        const ParFoot f = par_footprint(g, tab, x0, xn, y0, yn);
+        for (int h = f.lo; h <= f.hi; h++) {
+          // inside the staged span (see above); the clamp keeps the reads there
+          const int hh = max(min(h - slo, scnt - 1), 0);
+          double w;
+          const int use = par_weight(g, tab, f, hp_t[hh], w);
+          if (use == 0) continue;
+          if (use < 0) break;
+          add(rows_t + (size_t)hh * R, (float)w);
+        }
+      }
+    }
+    if (FOLD && group_ends && grp + 1 < ngrp) {
+      // running sum of the groups so far (the last group's is added below)
+      if (active) {
+#pragma unroll
+        for (int q = 0; q < R; q++)
+          if (q < nk) {
+            const Acc t = q < nrow ? acc[q] : (Acc)0;
+            vcol[q] = grp == 0 ? (float)t : (float)((Acc)vcol[q] + t);
+          }
+      }
 #pragma unroll
       for (int q = 0; q < R; q++) acc[q] = (Acc)0;
     }
-    for (int a0 = ga; a0 < gb; a0 += ab) {
-      const int nblk = min(ab, gb - a0);
-      if (tid < nblk) {
-        const CCPI_GLOBAL double *t = gmem(g.atab) + 5 * (a0 + tid);
-        const double c = t[0], s = t[1];
-        const double p0 = Y0 * c - X0 * s, p1 = YN * c - X0 * s;
-        const double p2 = Y0 * c - XN * s, p3 = YN * c - XN * s;
-        const double tmin = fmin(fmin(p0, p1), fmin(p2, p3));
-        const double tmax = fmax(fmax(p0, p1), fmax(p2, p3));
-        const int lo = max((int)floor(tmin * g.ihp - g.hp0) - 2, 0);
-        const int hi = min((int)floor(tmax * g.ihp - g.hp0) + 2, nh - 1);
-        s_lo[tid] = lo;
-        s_cnt[tid] = max(0, min(hi - lo + 1, hmax));
-      }
-      __syncthreads();
-      const int total = nblk * hmax * Q4;
-      for (int e = tid; e < total; e += 256) {
-        const int q4 = e % Q4, r = e / Q4;
-        const int hh = r % hmax, t = r / hmax;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (hh < s_cnt[t]) {
-          const CCPI_GLOBAL float *p =
-              gmem(sino) + ((size_t)(a0 + t) * nh + s_lo[t] + hh) * nv + k0 + 4 * q4;
-          if (aligned && 4 * q4 + 3 < nrow) {
-            v = load_f4(p);
-          } else {
-            if (4 * q4 < nrow) v.x = p[0];
-            if (4 * q4 + 1 < nrow) v.y = p[1];
-            if (4 * q4 + 2 < nrow) v.z = p[2];
-            if (4 * q4 + 3 < nrow) v.w = p[3];
-          }
-        }
-        *reinterpret_cast<float4 *>(s_rows + ((size_t)t * hmax + hh) * R + 4 * q4) = v;
-      }
-      __syncthreads();
-      if (active) {
-        for (int t = 0; t < nblk; t++) {
-          const int a = a0 + t;
-          const CCPI_GLOBAL double *tab = gmem(g.atab) + 5 * a;
-          const ParFoot f = par_footprint(g, tab, x0, xn, y0, yn);
-          const int slo = s_lo[t], scnt = s_cnt[t];
-          for (int h = f.lo; h <= f.hi; h++) {
-            double w;
-            const int use = par_weight(g, tab, f, gmem(g.h_pix)[h], w);
-            if (use == 0) continue;
-            if (use < 0) break;
-            const float wf = (float)w;
-            const int hh = h - slo;
-            if (hh >= 0 && hh < scnt) {
-              const float *pr = s_rows + ((size_t)t * hmax + hh) * R;
-#pragma unroll
-              for (int q4 = 0; q4 < Q4; q4++) {
-                const float4 v = *reinterpret_cast<const float4 *>(pr + 4 * q4);
-                acc[4 * q4] = acc[4 * q4] + (Acc)(v.x * wf);
-                acc[4 * q4 + 1] = acc[4 * q4 + 1] + (Acc)(v.y * wf);
-                acc[4 * q4 + 2] = acc[4 * q4 + 2] + (Acc)(v.z * wf);
-                acc[4 * q4 + 3] = acc[4 * q4 + 3] + (Acc)(v.w * wf);
-              }
-            } else {
-              const CCPI_GLOBAL float *pr = gmem(sino) + ((size_t)a * nh + h) * nv + k0;
-#pragma unroll
-              for (int q = 0; q < R; q++)
-                if (q < nrow) acc[q] = acc[q] + (Acc)(pr[q] * wf);
-            }
-          }
-        }
-      }
-      __syncthreads();
-    }
-    if (FOLD && active && grp + 1 < ngrp) {
-      // running sum of the groups so far (the last group's is added below)
-#pragma unroll
-      for (int q = 0; q < R; q++)
-        if (q < nk) vcol[q] = grp == 0 ? (float)acc[q] : (float)((Acc)vcol[q] + acc[q]);
-    }
+    if (!(next < next_gb)) break;
+    if (group_ends) grp++;
+    a0 = next;
+    gb = next_gb;
+    buf ^= 1;
   }
   if (!active) return 0.0;
   double ss = 0.0;
 #pragma unroll
   for (int q = 0; q < R; q++)
     if (q < nk) {
-      const float o =
-          (FOLD && groups > 1) ? (float)((Acc)vcol[q] + acc[q]) : (float)acc[q];
+      // slices without a row keep what they hold
+      float o;
+      if (FOLD && groups > 1)
+        o = (float)((Acc)vcol[q] + (q < nrow ? acc[q] : (Acc)0));
+      else
+        o = q < nrow ? (float)acc[q] : (!FOLD && acc_in ? vcol[q] : 0.0f);
       vcol[q] = o;
       ss += (double)o * (double)o;
     }

@@ -108,12 +108,11 @@ __global__ __launch_bounds__(256) void par_bp_kernel(ParArgs g,
 // The tiled BP as one launch: blockIdx.x = tile, y = slice chunk, z = angle
 // group; one group writes vol (adding to it when acc_in), several write
 // their partial sums to part[group] for par_bp_sum_kernel.  norm (one
-// group only): one partial of ||vol||^2 per workgroup.  The body waits on
-// its staged rows and footprints, not on issue: 5 waves per SIMD (94
-// VGPRs, a few spills in the set-up) instead of the 4 that 103 VGPRs allow
-// took the 64-problem mix's BP from 21.9 to 18.8 ms per round (6 waves:
-// 19.2), the 256 x 256 x 16 BP unchanged.  The FP64-accumulation instances
-// keep their registers.
+// group only): one partial of ||vol||^2 per workgroup.  5 waves per SIMD
+// (96 VGPRs, a few spills in the set-up): at 4 / 5 / 6 waves the
+// 512 x 512 x 32 BP takes 0.94 / 0.89 / 0.93 ms, 383 x 383 x 29 (ragged)
+// 0.39 / 0.31 / 0.33 and 256 x 256 x 16 0.079 / 0.081 / 0.090.  The
+// FP64-accumulation instances keep their registers.
 template <class Acc>
 constexpr int par_bp_lds_min_waves() { return std::is_same<Acc, float>::value ? 5 : 1; }
 
@@ -122,7 +121,7 @@ __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(par_bp_lds_min_waves<Acc>(), 8))) void par_bp_lds_kernel(
     ParArgs g, int hmax, int ab, int groups, const float *__restrict__ sino,
     float *__restrict__ vol, float *__restrict__ part, int acc_in, double *__restrict__ norm) {
-  extern __shared__ float smem[];
+  extern __shared__ __align__(16) float smem[];
   const int grp = blockIdx.z;
   const int a_begin = (int)((long long)g.na * grp / groups);
   const int a_end = (int)((long long)g.na * (grp + 1) / groups);
@@ -317,7 +316,7 @@ static ParTables par_tables(const Geometry &G, ParArgs &A) {
 
 // LDS of one tiled-BP workgroup: the staged rows and the per-angle spans.
 static size_t par_bp_lds_bytes(const ParBpShape &S) {
-  return sizeof(float) * (size_t)S.ab * S.hmax * S.slices + 2 * sizeof(int) * (size_t)S.ab;
+  return par_bp_tile_bytes(S.hmax, S.slices, S.ab);
 }
 
 // Shape of the tiled BP for a geometry, or tiled = 0.  The staged span of a
@@ -333,9 +332,8 @@ static ParBpShape par_bp_shape(const Geometry &G, const ParArgs &A) {
   const double span = std::hypot(16.0 * G.vsize[0], 16.0 * G.vsize[1]) * std::fabs(A.ihp);
   if (!(span < 4096.0)) return S;
   S.hmax = (int)std::ceil(span) + 6;
-  const size_t per_angle = sizeof(float) * (size_t)S.hmax * S.slices + 2 * sizeof(int);
-  if (per_angle > 32 * 1024) return S;
-  S.ab = (int)std::max<size_t>(1, std::min<size_t>(8, (32 * 1024) / per_angle));
+  if (sizeof(float) * (size_t)S.hmax * S.slices + 2 * sizeof(int) > 32 * 1024) return S;
+  S.ab = par_bp_block_angles(S.hmax, S.slices);
   const long long tiles = (long long)((G.nx + 15) / 16) * ((G.ny + 15) / 16);
   const long long waves = tiles * ((G.nz + S.slices - 1) / S.slices) * 4;
   S.groups = (int)std::min<long long>(std::min<long long>(8, G.na),
