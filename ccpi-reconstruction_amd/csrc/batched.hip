@@ -5,7 +5,7 @@
 // the iteration body is cgls_3d, Core/src/Algorithms/cgls.cpp:26-157).
 // Every step of an iteration is ONE launch over a flat work list that spans
 // all problems:
-//   FP    items (problem, 256/lr-ray block, 4*lr-row block) -> Ad, partial ||Ad||^2
+//   FP    items (problem, 64 rays of an angle, 4*lr-row block) -> Ad, partial ||Ad||^2
 //   alpha one workgroup per problem: fixed-order sum of its partials
 //   x/r   items (problem, element chunk)               -> x += a d, r -= a Ad
 //   BP    items (problem, 16x16-column tile or 256-column block, slice
@@ -17,10 +17,11 @@
 // problem descriptors in device memory, so a replay needs no host work.
 // The norms of the projector outputs are produced by the projector
 // epilogues (per work item, deterministic), so no separate reduction pass
-// re-reads Ad or s.  Rows-per-lane and, per projector, the grid (one
-// workgroup or wavefront per item, or a persistent grid of 2 / 4 / 8
-// workgroups per CU dealing the items out by a fixed stride) are picked by
-// timing candidates on the batch itself (autotune, cached per batch shape).
+// re-reads Ad or s.  The BP's rows per lane and grid (one workgroup per
+// item, or a persistent grid of 2 / 4 / 8 workgroups per CU dealing the items
+// out by a fixed stride) are picked by timing candidates on the batch itself
+// (autotune, cached per batch shape), and so is the grid of the FP items that
+// the shared walk does not take.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -49,6 +50,7 @@ struct BatchProb {
   float alpha, beta;
   int it;
   int fp_lr;           // FP lanes per ray
+  int fp_part, fp_parts;   // its norm partials: first and count
   int bp_tiled;        // BP items are 16 x 16 column tiles staged in LDS
   int bp_hmax, bp_ab;  // their staged detector columns per angle, angles per block
   int bp_groups;       // angle groups of the problem's one-problem tiled BP
@@ -56,11 +58,12 @@ struct BatchProb {
 
 struct BatchLists {
   int count;
-  const int *fp_off;   // [count + 1] item prefix per kernel type
+  const int *fs_off;   // [count + 1] item prefix per kernel type: shared-walk FP
+  const int *fp_off;   // other FP
   const int *bp_off;
   const int *vx_off;   // volume chunks
   const int *px_off;   // sinogram chunks
-  double *part_fp;     // [4 * fp items]: one per wave item
+  double *part_fp;     // one per live shared-walk item, 4 per other FP item
   double *part_bp;     // [4 * bp items]
 };
 
@@ -81,8 +84,41 @@ __device__ inline double wave_sum_d(double v) {
   return v;
 }
 
-// FP of d into Ad for every problem (mode 0), or BP of r into s (mode 1),
-// or BP of r into d (mode 2, initial direction).  FP work is taken per
+// FP of d into Ad for every problem whose rows and slices go one to one: one
+// workgroup per item, 64 rays of an angle walked by its first wavefront for
+// the other four (par_fp_shared), up to 8 lanes of 4 rows per ray.  Item
+// counts are multiples of 8 per problem, so an item's XCD is its place in its
+// problem's tiles (par_share_item).  With every lane walking on its own (the
+// form that batch_proj_kernel keeps for the other problems) an iteration of
+// the 64-problem mix took 27.8 ms, now 20.2 (7 waves per SIMD; 20.7 at 6).
+constexpr int kBatchShareThreads = 64 * 5, kBatchShareLanes = 8;
+
+__global__ __launch_bounds__(kBatchShareThreads)
+__attribute__((amdgpu_waves_per_eu(kParShareWavesPerSimd, 8))) void batch_fp_shared_kernel(
+    const BatchProb *__restrict__ P, BatchLists L) {
+  __shared__ ParShare sh;
+  const int p = find_prob(L.fs_off, L.count, blockIdx.x);
+  const BatchProb &B = P[p];
+  const ParArgs g = B.g;
+  const int lr = B.fp_lr;
+  const ParShareItem it = par_share_item(g, lr, (int)blockIdx.x - L.fs_off[p]);
+  if (!it.live) return;
+  const float *d = B.d;
+  float *Ad = B.Ad;
+  const int ns = lr == kBatchShareLanes ? 2 : 1;
+  double ss;
+  if (g.nz >= 4)
+    ss = ns == 2 ? par_fp_shared<2, true, float>(g, it.a, it.h0, it.v0, lr, d, Ad, false, sh)
+                 : par_fp_shared<1, true, float>(g, it.a, it.h0, it.v0, lr, d, Ad, false, sh);
+  else
+    ss = ns == 2 ? par_fp_shared<2, false, float>(g, it.a, it.h0, it.v0, lr, d, Ad, false, sh)
+                 : par_fp_shared<1, false, float>(g, it.a, it.h0, it.v0, lr, d, Ad, false, sh);
+  block_part(ss, L.part_fp, B.fp_part + it.index);
+}
+
+// FP of d into Ad for the problems that the shared walk does not take (mode
+// 0), or, for every problem, BP of r into s (mode 1) or into d (mode 2,
+// initial direction).  FP work is taken per
 // wavefront: a wave takes a block item (256 rays' lanes) and runs its four
 // 64-lane quarters in turn, so no wave waits at a barrier for the longest
 // walk of its workgroup.  BP work is taken per workgroup: a 16 x 16 column
@@ -126,7 +162,7 @@ __attribute__((amdgpu_waves_per_eu(batch_min_waves<MODE, BPK>(), 8))) void batch
         double ss = par_fp_lanes(g, local % B.fp_nbx, local / B.fp_nbx, qtr * 64 + lane,
                                  B.fp_lr, B.d, B.Ad, false);
         ss = wave_sum_d(ss);
-        if (lane == 0) part[4 * item + qtr] = ss;
+        if (lane == 0) part[B.fp_part + 4 * local + qtr] = ss;
       }
     }
     return;
@@ -161,11 +197,12 @@ template <int STEP>
 __global__ __launch_bounds__(256) void batch_scalar_kernel(BatchProb *__restrict__ P,
                                                            BatchLists L) {
   const int p = blockIdx.x;
-  const int *off = STEP == 1 ? L.fp_off : L.bp_off;
   const double *part = STEP == 1 ? L.part_fp : L.part_bp;
+  const int q0 = STEP == 1 ? P[p].fp_part : 4 * L.bp_off[p];
+  const int q1 = STEP == 1 ? q0 + P[p].fp_parts : 4 * L.bp_off[p + 1];
   __shared__ double sh[256];
   double s = 0.0;
-  for (int q = 4 * off[p] + threadIdx.x; q < 4 * off[p + 1]; q += 256) s += part[q];
+  for (int q = q0 + threadIdx.x; q < q1; q += 256) s += part[q];
   sh[threadIdx.x] = s;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
@@ -221,9 +258,9 @@ __global__ __launch_bounds__(256) void batch_vec_kernel(BatchProb *__restrict__ 
 
 namespace {
 
-// Launch shape of a batch: slices per BP item / rows per FP block (rc) and
-// the FP and BP grids: 0 launches one wavefront per FP item and one
-// workgroup per BP item (the dispatcher balances the uneven items), a
+// Launch shape of a batch: slices per BP item (rc) and the grids of the FP
+// items outside the shared walk and of the BP: 0 launches one wavefront per
+// FP item and one workgroup per BP item (the dispatcher balances the uneven items), a
 // positive value is a persistent grid of that many workgroups (capped at
 // residency) that deals the items out by a fixed stride.
 struct Tuned {
@@ -298,13 +335,19 @@ struct BatchRun {
   DeviceBuffer probs, offs, part_fp, part_bp, work, norms;
   BatchLists L{};
   int count = 0;
-  int fp_total = 0, bp_total = 0;
+  int fs_total = 0, fp_total = 0, bp_total = 0;
   size_t bp_lds = 0;   // dynamic LDS of the BP launches
   int bp_kinds = 0;    // BP bodies of the problems: 1 tiled, 2 column-per-lane
 };
 
 void proj(const BatchRun &R, const Tuned &T, int mode, hipStream_t st) {
   BatchProb *P = R.probs.as<BatchProb>();
+  if (mode == 0 && R.fs_total > 0) {
+    hipLaunchKernelGGL(batch_fp_shared_kernel, dim3((unsigned)R.fs_total),
+                       dim3(kBatchShareThreads), 0, st, P, R.L);
+    CCPI_HIP(hipGetLastError());
+  }
+  if (mode == 0 && R.fp_total == 0) return;
   const int grid = mode == 0 ? T.fp_grid : T.bp_grid;
   const int items = mode == 0 ? R.fp_total : R.bp_total;
   if (T.rc == 8)
@@ -318,7 +361,8 @@ void proj(const BatchRun &R, const Tuned &T, int mode, hipStream_t st) {
 // tiled BP gets tile items of rc slices, its staged span and angle groups
 // from the plan and its angles per staged block for rc slices.
 void layout(BatchRun &R, int rc, hipStream_t st) {
-  std::vector<int> off(4 * (R.count + 1), 0);
+  std::vector<int> off(5 * (R.count + 1), 0);
+  long long parts = 0;
   R.bp_lds = 0;
   R.bp_kinds = 0;
   for (int p = 0; p < R.count; p++) {
@@ -326,6 +370,8 @@ void layout(BatchRun &R, int rc, hipStream_t st) {
     const ParArgs &g = B.g;
     const ParBpShape &S = R.plans[p]->bp;
     B.fp_lr = par_fp_lanes_per_ray(g.nv);
+    const bool share = par_share_fits(g);
+    if (share) B.fp_lr = std::min(B.fp_lr, kBatchShareLanes);
     B.fp_nbx = (g.na * g.nh + 256 / B.fp_lr - 1) / (256 / B.fp_lr);
     B.fp_nby = (g.nv + 4 * B.fp_lr - 1) / (4 * B.fp_lr);
     B.bp_tiled = S.tiled;
@@ -340,7 +386,16 @@ void layout(BatchRun &R, int rc, hipStream_t st) {
       B.bp_nbx = (g.nx * g.ny + 255) / 256;
     }
     B.bp_nby = (g.nz + rc - 1) / rc;
-    off[p + 1] = off[p] + B.fp_nbx * B.fp_nby;
+    const long long fs = share ? par_share_items(g, B.fp_lr) : 0;
+    const long long fp = share ? 0 : (long long)B.fp_nbx * B.fp_nby;
+    B.fp_part = (int)parts;
+    B.fp_parts = share ? (int)par_share_parts(g, B.fp_lr) : (int)(4 * fp);
+    parts += B.fp_parts;
+    CCPI_REQUIRE(off[4 * (R.count + 1) + p] + fs < (1LL << 31) && off[p] + fp < (1LL << 31) &&
+                     parts < (1LL << 31),
+                 CCPI_E_LIMIT, "batched CGLS: too many rays");
+    off[p + 1] = off[p] + (int)fp;
+    off[4 * (R.count + 1) + p + 1] = off[4 * (R.count + 1) + p] + (int)fs;
     off[(R.count + 1) + p + 1] = off[(R.count + 1) + p] + B.bp_nbx * B.bp_nby;
     off[2 * (R.count + 1) + p + 1] =
         off[2 * (R.count + 1) + p] + (int)((B.nvox + kChunk - 1) / kChunk);
@@ -349,8 +404,9 @@ void layout(BatchRun &R, int rc, hipStream_t st) {
   }
   R.fp_total = off[R.count];
   R.bp_total = off[2 * R.count + 1];
+  R.fs_total = off[5 * R.count + 4];
   R.offs.upload(off, st);
-  R.part_fp.alloc((size_t)std::max(4 * R.fp_total, 1) * sizeof(double));  // per wave item
+  R.part_fp.alloc((size_t)std::max(parts, 1LL) * sizeof(double));
   R.part_bp.alloc((size_t)std::max(4 * R.bp_total, 1) * sizeof(double));
   int *o = R.offs.as<int>();
   R.L.count = R.count;
@@ -358,6 +414,7 @@ void layout(BatchRun &R, int rc, hipStream_t st) {
   R.L.bp_off = o + (R.count + 1);
   R.L.vx_off = o + 2 * (R.count + 1);
   R.L.px_off = o + 3 * (R.count + 1);
+  R.L.fs_off = o + 4 * (R.count + 1);
   R.L.part_fp = R.part_fp.as<double>();
   R.L.part_bp = R.part_bp.as<double>();
   R.probs.upload(R.host, st);

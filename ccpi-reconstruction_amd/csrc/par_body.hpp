@@ -495,6 +495,11 @@ struct ParWalker {
 // Volumes of the shared walk: their byte offsets, and the one an ended walk
 // asks for, stay below 2^32.
 constexpr size_t kParShareBytes = 0xe0000000;
+inline bool par_share_fits(const ParArgs &g) {
+  return g.map_type == 1 && sizeof(float) * (size_t)g.nx * g.ny * g.nz <= kParShareBytes;
+}
+// Waves per SIMD that the gathering wavefronts' registers allow (72 VGPRs).
+constexpr int kParShareWavesPerSimd = 7;
 
 // Adjacent angles that one XCD's consecutive workgroups take (16 / 32 / 64:
 // 512 x 512 x 32, 360 angles 0.739 / 0.720 / 0.720 ms, 383 x 383 x 29, 180
@@ -539,7 +544,7 @@ struct ParShare {
 };
 
 // Rows [v0, v0 + 4 lr) of rays h0 .. h0 + 63 of angle a, by a workgroup of
-// 1 + lr / NS wavefronts.  One row per slice, volumes below kParShareBytes
+// 1 + lr / NS wavefronts or more.  One row per slice, volumes below kParShareBytes
 // (32-bit byte offsets; the reads past the volume that a walk's end asks for
 // return 0).  VEC: nz >= 4, a lane's 4 slices in one 16-byte read that ends
 // inside the column; otherwise single reads.  Every thread of the workgroup
@@ -576,6 +581,13 @@ __device__ inline double par_fp_shared(const ParArgs &g, int a, int h0, int v0, 
   }
   const int per = 64 / lr;              // rays of one wavefront at a time
   const int ray0 = (wave - 1) * NS * per;
+  if (ray0 >= 64) {
+    // a wavefront more than the rays need: only the barriers
+    for (int buf = 0;; buf ^= 1) {
+      __syncthreads();
+      if (!__builtin_amdgcn_readfirstlane(sh.more[buf])) return 0.0;
+    }
+  }
   const int rl = lane & (lr - 1), rr = lane / lr;
   const int v = v0 + 4 * rl;            // the lane's first row
   const int nrow = max(0, min(4, g.nv - v)), nval = max(0, min(nrow, g.nz - v));

@@ -68,9 +68,6 @@ __global__ __launch_bounds__(256) void par_fp_table_kernel(ParArgs g, int lr,
   if (norm) block_part(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
 }
 
-#ifndef PFP_TA
-#define PFP_TA 64
-#endif
 // Workgroups of one XCD take the same 64 columns of kParTileA adjacent angles
 // (par_share_item): their rays cross mostly the same cells at the same time,
 // so the volume's columns are read from that XCD's L2 (512 x 512 x 32, 360
@@ -80,7 +77,9 @@ __global__ __launch_bounds__(256) void par_fp_table_kernel(ParArgs g, int lr,
 // 0.227, 256 x 256 x 16 0.079 / 0.088 / 0.080; the FP64-accumulation instances
 // keep their registers.
 template <class Acc>
-constexpr int par_fp_min_waves() { return std::is_same<Acc, float>::value ? 7 : 1; }
+constexpr int par_fp_min_waves() {
+  return std::is_same<Acc, float>::value ? kParShareWavesPerSimd : 1;
+}
 
 template <int NS, bool VEC, class Acc>
 __global__ __launch_bounds__(64 * (1 + 16 / 2))
@@ -407,8 +406,7 @@ enum class ParFpForm { kLanes, kTable, kShared };
 static ParFpForm par_fp_form(const ParArgs &A) {
   if (A.map_type != 1) return ParFpForm::kLanes;
   if (A.woff) return ParFpForm::kTable;
-  return sizeof(float) * (size_t)A.nx * A.ny * A.nz <= kParShareBytes ? ParFpForm::kShared
-                                                                     : ParFpForm::kLanes;
+  return par_share_fits(A) ? ParFpForm::kShared : ParFpForm::kLanes;
 }
 
 // Lanes per ray's cells of the table form: the most, up to 8, that keep
