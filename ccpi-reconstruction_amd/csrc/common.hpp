@@ -85,7 +85,8 @@ struct ConeArgs {
   int bp_unique;         // stride guarantees distinct slices per instruction
   int bp_main_safe;      // source inside the volume's z range
   int bp_phased;         // BP accumulates in one array, in lane phases
-  int bp_phases;         // lane phases (lanes of one phase on distinct slices)
+  int bp_rows;           // detector rows per lane of that form
+  int bp_phases;         // its lane phases (lanes of one phase on distinct slices)
   float bp_rps1;         // voxel z size / smallest row pitch: rows per slice at
                          // walk parameter 1
   int nvp;               // row stride of the BP's scaled sinogram (padded)

@@ -908,7 +908,7 @@ __device__ inline void bp_load_rows(__amdgpu_buffer_rsrc_t row, int at, int base
 // over distinct cells, issued together, followed by their second-slice
 // updates.  The kBpPad cells on each side of an array are trash for slices
 // outside the volume.  PHASED (rows per slice beyond 4, or arrays beyond
-// the LDS budget): S = 4, 8, 12 or 16 slots and one array; the slots update
+// the LDS budget): S slots (1 to 16) and one array; the slots update
 // one after another, each in read-add-write rounds, and within a slot the
 // lanes go in phases (lane L in phase L mod phases), whose lanes are
 // phases * S >= rows per slice rows apart, so on distinct slices.  The
@@ -962,22 +962,21 @@ __device__ void bp_phased_block(const ConeArgs &g, const BpRec *__restrict__ R, 
     dzv[t] = g.dz[vv];
     izv[t] = g.iz[vv];
   }
-  static_assert(S % 4 == 0, "the phased form loads 4 rows at a time");
   auto live = [&](const BpRec &rec) {
     return vb < (int)(rec.w >> 16) && vb + span > (int)(rec.w & 0xffffu);
   };
   auto gather = [&](const BpRec &rec, float *p) {
-    // rows vlane .. vlane + S - 1 of the record's padded row, 16 bytes per
-    // load (nvp is a multiple of 64 * S, so every row is in range; one
+    // rows vlane .. vlane + S - 1 of the record's padded row, up to 16 bytes
+    // per load (nvp is a multiple of 64 * S, so every row is in range; one
     // dword per load made the wide-cone BP 1.8x slower)
-    const float4 *src = (const float4 *)(dpix + (size_t)rec.x * g.nvp + vlane);
+    constexpr int W = S % 4 == 0 ? 4 : (S % 3 == 0 ? 3 : S);
+    struct Rows { float r[W]; };
+    const Rows *src = (const Rows *)(dpix + (size_t)rec.x * g.nvp + vlane);
 #pragma unroll
-    for (int j = 0; j < S / 4; ++j) {
-      const float4 q = src[j];
-      p[4 * j] = q.x;
-      p[4 * j + 1] = q.y;
-      p[4 * j + 2] = q.z;
-      p[4 * j + 3] = q.w;
+    for (int j = 0; j < S / W; ++j) {
+      const Rows q = src[j];
+#pragma unroll
+      for (int w = 0; w < W; ++w) p[W * j + w] = q.r[w];
     }
   };
   auto update = [&](const BpRec &rec, const float *p, int pass, auto MAIN, auto ONE) {
@@ -1482,10 +1481,23 @@ BpLayout cone_bp_layout(const Geometry &G) {
     }
     L.phases = phases(L.stride);
   }
+  // A lane takes fewer rows, in as many more phases, where the detector's
+  // rows would leave lanes idle: the least of 1, 2, 3, 4, 6, 8, 12 that covers
+  // them in one block.  Wide cones, S = 8 before (ms per BP): 128 rows, S = 2
+  // 0.685 -> 0.505; 192, S = 3 1.84 -> 1.74; 240, S = 4 3.75 -> 3.23; 300,
+  // S = 6 7.59 -> 6.34; 384, S = 6 16.3 -> 13.5.  Over more than one block it
+  // does not pay: 448 rows with S = 4 33.7, 600 with S = 6 (S = 12 before)
+  // 58.4 -> 63.3.
+  L.rows = L.stride;
+  if (L.phased) {
+    for (int S : {12, 8, 6, 4, 3, 2, 1})
+      if (S < L.rows && 64 * S >= nv) L.rows = S;
+    L.row_phases = std::min(64, (want + L.rows - 1) / L.rows);
+  }
   CCPI_REQUIRE(bp_lds_bytes(nz, L.phased ? 1 : L.stride) <= 160 * 1024, CCPI_E_LIMIT,
                "cone BP: nz too large for LDS");
-  // rows of one BP block: 64 lanes bp_stride rows apart (both forms)
-  const int span = 64 * L.stride;
+  // rows of one BP block: 64 lanes `rows` apart (both forms)
+  const int span = 64 * L.rows;
   L.nvp = (nv + span - 1) / span * span;
   CCPI_REQUIRE(nv < 65536, CCPI_E_LIMIT, "cone beam: at most 65535 detector rows");
   L.want = want;
@@ -1595,7 +1607,8 @@ void cone_build_plan(ConePlan &P, hipStream_t st) {
     A.bp_unique = L.unique;
     A.bp_main_safe = L.main_safe;
     A.bp_phased = L.phased;
-    A.bp_phases = L.phases;
+    A.bp_rows = L.rows;
+    A.bp_phases = L.row_phases;
     A.bp_rps1 = (float)L.rps1;
     A.nvp = L.nvp;
   }
@@ -1781,19 +1794,22 @@ static void cone_bp_launch(const ConePlan &P, const float *dpix, float *vol, hip
   const BpCol *bc = P.bpcol.as<BpCol>();
   const BpRec *br = P.bprec.as<BpRec>();
   const dim3 grid(blocks), block(64 * kBpWaves);
-  if (A.bp_phased && A.bp_stride == 4)
-    hipLaunchKernelGGL((cone_bp_kernel<4, true, AccT>), grid, block, lds, st, A, bc, br, dpix,
-                       vol, ai, norm);
-  else if (A.bp_phased && A.bp_stride == 8)
-    hipLaunchKernelGGL((cone_bp_kernel<8, true, AccT>), grid, block, lds, st, A, bc, br, dpix,
-                       vol, ai, norm);
-  else if (A.bp_phased && A.bp_stride == 12)
-    hipLaunchKernelGGL((cone_bp_kernel<12, true, AccT>), grid, block, lds, st, A, bc, br, dpix,
-                       vol, ai, norm);
-  else if (A.bp_phased)
-    hipLaunchKernelGGL((cone_bp_kernel<16, true, AccT>), grid, block, lds, st, A, bc, br, dpix,
-                       vol, ai, norm);
-  else if (narr == 1)
+  if (A.bp_phased) {
+    auto go = [&](auto S) {
+      hipLaunchKernelGGL((cone_bp_kernel<decltype(S)::value, true, AccT>), grid, block, lds, st, A,
+                         bc, br, dpix, vol, ai, norm);
+    };
+    switch (A.bp_rows) {
+      case 1: go(std::integral_constant<int, 1>{}); break;
+      case 2: go(std::integral_constant<int, 2>{}); break;
+      case 3: go(std::integral_constant<int, 3>{}); break;
+      case 4: go(std::integral_constant<int, 4>{}); break;
+      case 6: go(std::integral_constant<int, 6>{}); break;
+      case 8: go(std::integral_constant<int, 8>{}); break;
+      case 12: go(std::integral_constant<int, 12>{}); break;
+      default: go(std::integral_constant<int, 16>{}); break;
+    }
+  } else if (narr == 1)
     hipLaunchKernelGGL((cone_bp_kernel<1, false, AccT>), grid, block, lds, st, A, bc, br, dpix,
                        vol, ai, norm);
   else if (narr == 2)

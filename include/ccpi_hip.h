@@ -206,7 +206,8 @@ int ccpi_pb_cgls_batched(const ccpi_geometry *geoms, int count,
 /* BP accumulation layout the library picks for a cone geometry, computed
    on the host only (no device work, usable without a GPU): *row_stride =
    detector rows per lane (S), *phased = 1 for the one-array form whose
-   lanes update in *phases rounds, *rows_bound = the bound on detector rows
+   lanes update in *phases rounds (with fewer rows per lane in as many more
+   rounds for a detector of fewer than 64 * S rows), *rows_bound = the bound on detector rows
    per voxel slice over all columns that the choice guarantees (lanes of one
    round are >= that many rows apart, or alone in their round).  No
    counterpart in the reference: its b2D accumulates each voxel column on
