@@ -330,9 +330,9 @@ struct BatchRun;
 void proj(const BatchRun &R, const Tuned &T, int mode, hipStream_t st);
 
 struct BatchRun {
-  std::vector<std::shared_ptr<ParPlan>> plans;
+  Workspace &W;
+  ParBatchPlan plan;
   std::vector<BatchProb> host;
-  DeviceBuffer probs, offs, part_fp, part_bp, work, norms;
   BatchLists L{};
   int count = 0;
   int fs_total = 0, fp_total = 0, bp_total = 0;
@@ -341,7 +341,7 @@ struct BatchRun {
 };
 
 void proj(const BatchRun &R, const Tuned &T, int mode, hipStream_t st) {
-  BatchProb *P = R.probs.as<BatchProb>();
+  BatchProb *P = R.W.probs.as<BatchProb>();
   if (mode == 0 && R.fs_total > 0) {
     hipLaunchKernelGGL(batch_fp_shared_kernel, dim3((unsigned)R.fs_total),
                        dim3(kBatchShareThreads), 0, st, P, R.L);
@@ -368,7 +368,7 @@ void layout(BatchRun &R, int rc, hipStream_t st) {
   for (int p = 0; p < R.count; p++) {
     BatchProb &B = R.host[p];
     const ParArgs &g = B.g;
-    const ParBpShape &S = R.plans[p]->bp;
+    const ParBpShape &S = R.plan.bp[p];
     B.fp_lr = par_fp_lanes_per_ray(g.nv);
     const bool share = par_share_fits(g);
     if (share) B.fp_lr = std::min(B.fp_lr, kBatchShareLanes);
@@ -405,19 +405,19 @@ void layout(BatchRun &R, int rc, hipStream_t st) {
   R.fp_total = off[R.count];
   R.bp_total = off[2 * R.count + 1];
   R.fs_total = off[5 * R.count + 4];
-  R.offs.upload(off, st);
-  R.part_fp.alloc((size_t)std::max(parts, 1LL) * sizeof(double));
-  R.part_bp.alloc((size_t)std::max(4 * R.bp_total, 1) * sizeof(double));
-  int *o = R.offs.as<int>();
+  R.W.offs.upload(off, st);
+  R.W.part.alloc((size_t)std::max(parts, 1LL) * sizeof(double));
+  R.W.part2.alloc((size_t)std::max(4 * R.bp_total, 1) * sizeof(double));
+  int *o = R.W.offs.as<int>();
   R.L.count = R.count;
   R.L.fp_off = o;
   R.L.bp_off = o + (R.count + 1);
   R.L.vx_off = o + 2 * (R.count + 1);
   R.L.px_off = o + 3 * (R.count + 1);
   R.L.fs_off = o + 4 * (R.count + 1);
-  R.L.part_fp = R.part_fp.as<double>();
-  R.L.part_bp = R.part_bp.as<double>();
-  R.probs.upload(R.host, st);
+  R.L.part_fp = R.W.part.as<double>();
+  R.L.part_bp = R.W.part2.as<double>();
+  R.W.probs.upload(R.host, st);
 }
 
 int cu_count() {
@@ -431,7 +431,9 @@ int cu_count() {
 
 void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
                          float *const *x, int iters, double *norms_out, hipStream_t caller) {
-  BatchRun R;
+  WorkspaceLease lease;
+  std::vector<char> tables;
+  BatchRun R{*lease};
   R.count = (int)geoms.size();
   if (R.count == 0) return;
   CCPI_HIP(hipStreamSynchronize(caller));
@@ -445,20 +447,19 @@ void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
   // per-problem work vectors carved from one allocation
   size_t total = 0;
   for (const Geometry &G : geoms) total += 2 * G.n_vox() + G.n_pix();
-  R.work.alloc(total * sizeof(float));
-  R.norms.alloc((size_t)R.count * std::max(iters, 1) * sizeof(double));
-  float *w = R.work.as<float>();
+  R.W.v1.alloc(total * sizeof(float));
+  R.W.norms.alloc((size_t)R.count * std::max(iters, 1) * sizeof(double));
+  float *w = R.W.v1.as<float>();
+  for (const Geometry &G : geoms)
+    CCPI_REQUIRE(G.kind == CCPI_PARALLEL, CCPI_E_ARG, "batched CGLS takes parallel-beam problems");
+  // no plans: 64 problems would go through a cache of 8, each with uploads of
+  // its own and, for the small ones, a walk table that a batch does not use
+  R.plan = par_batch_plan(geoms, tables, R.W.tabs, st);
   std::string sig;
   for (int p = 0; p < R.count; p++) {
     const Geometry &G = geoms[p];
-    CCPI_REQUIRE(G.kind == CCPI_PARALLEL, CCPI_E_ARG, "batched CGLS takes parallel-beam problems");
-    R.plans.push_back(par_plan(G, st));
     BatchProb B{};
-    B.g = R.plans.back()->args;
-    // the one launch holds every problem's rays: the FP walks them (a walk
-    // table's dependent load would lengthen the gathers' latency chain)
-    B.g.woff = nullptr;
-    B.g.went = nullptr;
+    B.g = R.plan.args[p];
     B.r = b[p];
     B.x = x[p];
     B.d = w;
@@ -467,7 +468,7 @@ void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
     w += G.n_vox();
     B.Ad = w;
     w += G.n_pix();
-    B.norms = R.norms.as<double>() + (size_t)p * std::max(iters, 1);
+    B.norms = R.W.norms.as<double>() + (size_t)p * std::max(iters, 1);
     B.nvox = (long long)G.n_vox();
     B.npix = (long long)G.n_pix();
     R.host.push_back(B);
@@ -543,7 +544,7 @@ void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
     g_tuned[sig] = T;
   }
   layout(R, T.rc, st);
-  BatchProb *P = R.probs.as<BatchProb>();
+  BatchProb *P = R.W.probs.as<BatchProb>();
   const int vgrid = 4 * cu_count();
 
   // start: d = A^T b, gamma = ||d||^2 (cgls.cpp:45-49)
@@ -574,9 +575,10 @@ void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
   gg.e = exec;
   for (int it = 0; it < iters; it++) CCPI_HIP(hipGraphLaunch(exec, st));
   if (norms_out && iters > 0)
-    CCPI_HIP(hipMemcpyAsync(norms_out, R.norms.p, (size_t)R.count * iters * sizeof(double),
+    CCPI_HIP(hipMemcpyAsync(norms_out, R.W.norms.p, (size_t)R.count * iters * sizeof(double),
                             hipMemcpyDeviceToHost, st));
   CCPI_HIP(hipStreamSynchronize(st));
+  lease.keep();
 }
 
 }  // namespace ccpi

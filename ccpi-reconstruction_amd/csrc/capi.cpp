@@ -130,10 +130,11 @@ int ccpi_cgls(const ccpi_geometry *g, float *b, float *x, int iterations, double
     CCPI_REQUIRE(b && x, CCPI_E_ARG, "null data pointer");
     CCPI_REQUIRE(iterations >= 0, CCPI_E_ARG, "negative iteration count");
     ccpi::Projector P(ccpi::Geometry::from(g), S(stream));
-    ccpi::Workspace W;
-    ccpi::run_cgls(P, b, x, iterations, norms, (flags & CCPI_REDUCE_FP32) != 0, W,
+    ccpi::WorkspaceLease W;
+    ccpi::run_cgls(P, b, x, iterations, norms, (flags & CCPI_REDUCE_FP32) != 0, *W,
                    S(stream));
     CCPI_HIP(hipStreamSynchronize(S(stream)));
+    W.keep();
   });
 }
 
@@ -145,11 +146,13 @@ int ccpi_regularize(int kind, const float *a, float *out, int nx, int ny, int nz
     CCPI_REQUIRE(kind == CCPI_REG_TIKHONOV || kind == CCPI_REG_TV, CCPI_E_ARG,
                  "unknown regularisation kind");
     ccpi::check_reg_dims(nx, ny, nz);
-    ccpi::DeviceBuffer scr;
+    ccpi::WorkspaceLease W;
+    ccpi::DeviceBuffer &scr = (*W).tvd;
     const size_t nscr = ccpi::reg_scratch_floats(kind, (size_t)nx * ny * nz);
     if (nscr) scr.alloc(nscr * sizeof(float));
     ccpi::reg_term(kind, a, out, nscr ? scr.as<float>() : nullptr, nx, ny, nz, S(stream));
     CCPI_HIP(hipStreamSynchronize(S(stream)));
+    W.keep();
   });
 }
 
@@ -161,9 +164,10 @@ int ccpi_cgls_reg(const ccpi_geometry *g, float *b, float *x, int iterations, in
     CCPI_REQUIRE(kind == CCPI_REG_TIKHONOV || kind == CCPI_REG_TV, CCPI_E_ARG,
                  "unknown regularisation kind");
     ccpi::Projector P(ccpi::Geometry::from(g), S(stream));
-    ccpi::Workspace W;
+    ccpi::WorkspaceLease W;
     ccpi::run_cgls_reg(P, b, x, iterations, kind, lambda, norms,
-                       (flags & CCPI_REDUCE_FP32) != 0, W, S(stream));
+                       (flags & CCPI_REDUCE_FP32) != 0, *W, S(stream));
+    W.keep();
   });
 }
 
@@ -183,9 +187,10 @@ int ccpi_sirt(const ccpi_geometry *g, const float *b, float *x, int iterations, 
     CCPI_REQUIRE(b && x, CCPI_E_ARG, "null data pointer");
     CCPI_REQUIRE(iterations >= 0, CCPI_E_ARG, "negative iteration count");
     ccpi::Projector P(ccpi::Geometry::from(g), S(stream));
-    ccpi::Workspace W;
-    ccpi::run_sirt(P, b, x, iterations, W, S(stream));
+    ccpi::WorkspaceLease W;
+    ccpi::run_sirt(P, b, x, iterations, *W, S(stream));
     CCPI_HIP(hipStreamSynchronize(S(stream)));
+    W.keep();
   });
 }
 
@@ -196,9 +201,10 @@ int ccpi_mlem(const ccpi_geometry *g, const float *b, float *x, int iterations, 
     CCPI_REQUIRE(b && x, CCPI_E_ARG, "null data pointer");
     CCPI_REQUIRE(iterations >= 0, CCPI_E_ARG, "negative iteration count");
     ccpi::Projector P(ccpi::Geometry::from(g), S(stream));
-    ccpi::Workspace W;
-    ccpi::run_mlem(P, b, x, iterations, W, S(stream), (flags & CCPI_ACCUM_FP64) != 0);
+    ccpi::WorkspaceLease W;
+    ccpi::run_mlem(P, b, x, iterations, *W, S(stream), (flags & CCPI_ACCUM_FP64) != 0);
     CCPI_HIP(hipStreamSynchronize(S(stream)));
+    W.keep();
   });
 }
 
@@ -253,7 +259,7 @@ int ccpi_cgls_norms(ccpi_cgls_state *s, double *norms, int *done) {
   return guarded([&] {
     CCPI_REQUIRE(s, CCPI_E_ARG, "null session");
     if (norms && s->done > 0) {
-      CCPI_HIP(hipMemcpyAsync(norms, s->run.norms_dev.p, (size_t)s->done * sizeof(double),
+      CCPI_HIP(hipMemcpyAsync(norms, s->W.norms.p, (size_t)s->done * sizeof(double),
                               hipMemcpyDeviceToHost, s->st));
     }
     CCPI_HIP(hipStreamSynchronize(s->st));

@@ -391,6 +391,38 @@ void par_build_plan(ParPlan &P, hipStream_t st) {
   P.bp = par_bp_shape(G, A);
 }
 
+ParBatchPlan par_batch_plan(const std::vector<Geometry> &gs, std::vector<char> &img,
+                            DeviceBuffer &dev, hipStream_t st) {
+  ParBatchPlan B;
+  struct At { size_t atab, hpix, map, rlo, rhi; };
+  std::vector<At> at;
+  img.clear();
+  auto put = [&](const auto &v) {
+    const size_t o = img.size(), n = v.size() * sizeof(v[0]);
+    img.resize(o + (n + 15) / 16 * 16);
+    std::memcpy(img.data() + o, v.data(), n);
+    return o;
+  };
+  for (const Geometry &G : gs) {
+    ParArgs A;
+    const ParTables T = par_tables(G, A);
+    at.push_back({put(T.atab), put(G.h_pix), put(T.map), put(T.rlo), put(T.rhi)});
+    B.args.push_back(A);
+    B.bp.push_back(par_bp_shape(G, A));
+  }
+  dev.upload(img, st);
+  char *p = dev.as<char>();
+  for (size_t q = 0; q < gs.size(); q++) {
+    ParArgs &A = B.args[q];
+    A.atab = (const double *)(p + at[q].atab);
+    A.h_pix = (const double *)(p + at[q].hpix);
+    A.map = (const int *)(p + at[q].map);
+    A.rlo = (const int *)(p + at[q].rlo);
+    A.rhi = (const int *)(p + at[q].rhi);
+  }
+  return B;
+}
+
 // How the FP of a geometry runs.
 enum class ParFpForm { kLanes, kTable, kShared };
 

@@ -247,6 +247,7 @@ std::shared_ptr<ParPlan> par_plan(const Geometry &g, hipStream_t st) {
 }
 
 void plan_cache_clear() {
+  workspaces_give_back();
   Cache &c = cache();
   std::lock_guard<std::mutex> lock(c.mu);
   c.lru.clear();

@@ -47,6 +47,9 @@ struct Geometry {
 };
 
 // Owning device allocation.
+// Frees the workspaces that calls have left for the next (solvers.hip).
+void workspaces_give_back();
+
 struct DeviceBuffer {
   void *p = nullptr;
   size_t bytes = 0;
@@ -62,7 +65,12 @@ struct DeviceBuffer {
   void alloc(size_t n) {
     if (n <= bytes && p) return;
     reset();
-    CCPI_HIP(hipMalloc(&p, n ? n : 4));
+    if (hipMalloc(&p, n ? n : 4) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      workspaces_give_back();
+      CCPI_HIP(hipMalloc(&p, n ? n : 4));
+    }
     bytes = n;
   }
   template <class T>
@@ -230,6 +238,14 @@ void par_build_plan(ParPlan &P, hipStream_t st);
 // a fixed file-scope device array of kNoAllocScratchBytes (parallel.hip).
 constexpr size_t kNoAllocScratchBytes = size_t(1) << 20;
 size_t par_noalloc_bytes(const Geometry &g);
+// Arguments and BP shapes of several geometries without walk tables, their
+// tables in `dev` in one copy from `img` (which has to outlive it).
+struct ParBatchPlan {
+  std::vector<ParArgs> args;
+  std::vector<ParBpShape> bp;
+};
+ParBatchPlan par_batch_plan(const std::vector<Geometry> &gs, std::vector<char> &img,
+                            DeviceBuffer &dev, hipStream_t st);
 void par_fp_noalloc(const Geometry &g, const float *vol, float *sino, hipStream_t st);
 void par_fp(const ParPlan &P, const float *vol, float *sino, hipStream_t st, bool f64 = false,
             bool acc_in = true, double *norm = nullptr);

@@ -15,6 +15,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <list>
+#include <memory>
+#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -312,6 +315,66 @@ void dev_fill(float *p, size_t n, float v, hipStream_t st) {
 
 Workspace::~Workspace() = default;
 
+size_t Workspace::bytes() const {
+  size_t b = 0;
+  for (const DeviceBuffer *q : {&v1, &v2, &v3, &p1, &p2, &part, &fold, &scal, &v4, &part2, &tvd,
+                                &dscale, &norms, &offs, &probs, &tabs})
+    b += q->bytes;
+  return b;
+}
+
+namespace {
+struct KeptWorkspaces {
+  std::mutex mu;
+  std::list<std::pair<int, std::unique_ptr<Workspace>>> idle;   // (device, workspace), last left first
+};
+KeptWorkspaces &kept() {
+  static KeptWorkspaces k;
+  return k;
+}
+}  // namespace
+
+WorkspaceLease::WorkspaceLease() {
+  CCPI_HIP(hipGetDevice(&dev_));
+  KeptWorkspaces &k = kept();
+  {
+    std::lock_guard<std::mutex> lk(k.mu);
+    for (auto it = k.idle.begin(); it != k.idle.end(); ++it)
+      if (it->first == dev_) {
+        w_ = std::move(it->second);
+        k.idle.erase(it);
+        return;
+      }
+  }
+  w_ = std::make_unique<Workspace>();
+}
+
+WorkspaceLease::~WorkspaceLease() {
+  if (!keep_ || w_->bytes() > kKeptBytes) return;
+  KeptWorkspaces &k = kept();
+  std::list<std::pair<int, std::unique_ptr<Workspace>>> over;   // freed outside the lock
+  std::lock_guard<std::mutex> lk(k.mu);
+  k.idle.emplace_front(dev_, std::move(w_));
+  size_t n = 0, b = 0;
+  for (auto it = k.idle.begin(); it != k.idle.end();) {
+    const auto q = it++;
+    n++;
+    b += q->second->bytes();
+    if (n > kKeptWorkspaces || b > kKeptBytes) {
+      b -= q->second->bytes();
+      n--;
+      over.splice(over.end(), k.idle, q);
+    }
+  }
+}
+
+void workspaces_give_back() {
+  std::list<std::pair<int, std::unique_ptr<Workspace>>> all;
+  KeptWorkspaces &k = kept();
+  std::lock_guard<std::mutex> lk(k.mu);
+  all.swap(k.idle);
+}
+
 void Workspace::ensure(const Projector &P) {
   const size_t nvox = P.geometry().n_vox(), npix = P.geometry().n_pix();
   if (const size_t nd = P.bp_scratch_floats()) dscale.alloc(nd * 4);
@@ -350,7 +413,7 @@ static void sumsq(const float *x, size_t n, void *part, hipStream_t st) {
 void CglsRun::start(hipStream_t st) {
   const size_t nvox = P.geometry().n_vox();
   W.ensure(P);
-  norms_dev.alloc((size_t)std::max(iters, 1) * sizeof(double));
+  W.norms.alloc((size_t)std::max(iters, 1) * sizeof(double));
   float *d = W.v1.as<float>();
   if (fp32) {
     // the reference's float partial sums: a separate pass over d
@@ -439,12 +502,12 @@ void CglsRun::iterate(int it, hipStream_t st) {
   if (fp32) {
     sumsq<float>(s, nvox, W.part.p, st);
     hipLaunchKernelGGL(cgls_beta_kernel<float>, dim3(1), dim3(kRedThreads), 0, st,
-                       W.part.as<float>(), kRedBlocks, sc, norms_dev.as<double>(), it, 1);
+                       W.part.as<float>(), kRedBlocks, sc, W.norms.as<double>(), it, 1);
   } else {
     size_t n = P.bp_norm_parts();
     const double *pp = fold_parts(W.part.as<double>(), n, W.fold.as<double>(), st);
     hipLaunchKernelGGL(cgls_beta_kernel<double>, dim3(1), dim3(kRedThreads), 0, st, pp, (int)n,
-                       sc, norms_dev.as<double>(), it, 0);
+                       sc, W.norms.as<double>(), it, 0);
   }
   hipLaunchKernelGGL(cgls_update_d_kernel, dim3(grid_for(nvox)), dim3(256), 0, st, d, s, nvox,
                      sc);
@@ -453,7 +516,7 @@ void CglsRun::iterate(int it, hipStream_t st) {
 
 void CglsRun::finish(double *norms, hipStream_t st) {
   if (norms && iters > 0) {
-    CCPI_HIP(hipMemcpyAsync(norms, norms_dev.p, (size_t)iters * sizeof(double),
+    CCPI_HIP(hipMemcpyAsync(norms, W.norms.p, (size_t)iters * sizeof(double),
                             hipMemcpyDeviceToHost, st));
     CCPI_HIP(hipStreamSynchronize(st));
   }
@@ -483,8 +546,7 @@ void run_cgls_reg(const Projector &P, float *b, float *x, int iters, int kind, d
   W.part2.alloc(kRedBlocks * sizeof(double));
   const size_t nscr = reg_scratch_floats(kind, nvox);
   if (nscr) W.tvd.alloc(nscr * 4);
-  DeviceBuffer norms_dev;
-  norms_dev.alloc((size_t)std::max(iters, 1) * sizeof(double));
+  W.norms.alloc((size_t)std::max(iters, 1) * sizeof(double));
   float *d = W.v1.as<float>(), *s = W.v2.as<float>(), *L = W.v3.as<float>();
   float *adv = W.v4.as<float>(), *Ad = W.p1.as<float>();
   float *scr = nscr ? W.tvd.as<float>() : nullptr;
@@ -536,18 +598,18 @@ void run_cgls_reg(const Projector &P, float *b, float *x, int iters, int kind, d
     if (fp32) {
       sumsq<float>(s, nvox, W.part.p, st);
       hipLaunchKernelGGL(cgls_beta_kernel<float>, dim3(1), dim3(kRedThreads), 0, st,
-                         W.part.as<float>(), kRedBlocks, sc, norms_dev.as<double>(), it, 1);
+                         W.part.as<float>(), kRedBlocks, sc, W.norms.as<double>(), it, 1);
     } else {
       size_t n = P.bp_norm_parts();
       const double *pp = fold_parts(W.part.as<double>(), n, W.fold.as<double>(), st);
       hipLaunchKernelGGL(cgls_beta_kernel<double>, dim3(1), dim3(kRedThreads), 0, st, pp,
-                         (int)n, sc, norms_dev.as<double>(), it, 0);
+                         (int)n, sc, W.norms.as<double>(), it, 0);
     }
     hipLaunchKernelGGL(cgls_update_d_kernel, dim3(gv), dim3(256), 0, st, d, s, nvox, sc);
     CCPI_HIP(hipGetLastError());
   }
   if (norms && iters > 0) {
-    CCPI_HIP(hipMemcpyAsync(norms, norms_dev.p, (size_t)iters * sizeof(double),
+    CCPI_HIP(hipMemcpyAsync(norms, W.norms.p, (size_t)iters * sizeof(double),
                             hipMemcpyDeviceToHost, st));
   }
   CCPI_HIP(hipStreamSynchronize(st));

@@ -1,6 +1,7 @@
 // Device-resident iteration bodies (see solvers.hip).
 #pragma once
 
+#include <memory>
 #include <vector>
 
 #include "plan.hpp"
@@ -26,10 +27,35 @@ struct Workspace {
   DeviceBuffer v4, part2;    // regularised CGLS: Ad_vox, its partials
   DeviceBuffer tvd;          // TV term: D1, D2, D3
   DeviceBuffer dscale;       // cone BP input scaled by d_conv (padded rows)
+  DeviceBuffer norms;        // ||A^T r|| per iteration
+  DeviceBuffer offs, probs, tabs;   // batched CGLS: item lists, problems, their tables
   ~Workspace();
+  size_t bytes() const;
   void ensure(const Projector &P);
   // the workspace's BP scratch (nullptr when the projector needs none)
   float *bp_scratch() const { return dscale.p ? dscale.as<float>() : nullptr; }
+};
+
+// A workspace for one call: one that an earlier call of this device left, or
+// a new one.  A call that ends with its stream synchronised leaves it for the
+// next (keep()); kKeptWorkspaces of them and kKeptBytes at most stay, until
+// plan_cache_clear or until the device runs out of memory.  Allocating and
+// freeing them on each call took 0.2 to 0.5 ms.
+constexpr size_t kKeptWorkspaces = 4, kKeptBytes = size_t(2) << 30;
+class WorkspaceLease {
+ public:
+  WorkspaceLease();
+  ~WorkspaceLease();
+  WorkspaceLease(const WorkspaceLease &) = delete;
+  WorkspaceLease &operator=(const WorkspaceLease &) = delete;
+  Workspace &operator*() { return *w_; }
+  // the device has finished with the workspace
+  void keep() { keep_ = true; }
+
+ private:
+  std::unique_ptr<Workspace> w_;
+  int dev_ = 0;
+  bool keep_ = false;
 };
 
 // regularize.hip: Tikhonov / TV terms (tikhonov.cpp, total_v.cpp)
@@ -58,7 +84,6 @@ struct CglsRun {
   float *x;      // volume in/out
   int iters;
   bool fp32;
-  DeviceBuffer norms_dev;
   EventLog *log = nullptr;
   void start(hipStream_t st);
   void iterate(int it, hipStream_t st);

@@ -221,7 +221,9 @@ const char *ccpi_error_string(int status);
    successful call). */
 const char *ccpi_last_error(void);
 int ccpi_version(void);
-/* Drop cached per-geometry plans (device tables) on the current device. */
+/* Drop cached per-geometry plans (device tables) on the current device, and
+   the workspaces that solver calls have left for the next one (at most four,
+   2 GiB together, not counted by ccpi_plan_cache_bytes). */
 void ccpi_plan_cache_clear(void);
 /* Device bytes held by cached plans on the current device. */
 long long ccpi_plan_cache_bytes(void);
