@@ -282,6 +282,14 @@ __device__ inline uint32_t k4_add(int k, uint32_t base) {
   asm("v_lshl_add_u32 %0, %1, 2, %2" : "=v"(r) : "v"(k), "v"(base));
   return r;
 }
+// base + k cells of T
+template <class T>
+__device__ inline uint32_t cell_add(int k, uint32_t base) {
+  if constexpr (sizeof(T) == 4) return k4_add(k, base);
+  uint32_t r;
+  asm("v_lshl_add_u32 %0, %1, 3, %2" : "=v"(r) : "v"(k), "v"(base));
+  return r;
+}
 
 // min(a, b) for a uniform a as one v_min_f32 (the select form needs a
 // copy of a into a VGPR); operands are finite alphas, so this is the
@@ -1078,8 +1086,9 @@ __device__ void bp_phased_block(const ConeArgs &g, const BpRec *__restrict__ R, 
 
 // AccT is the type of the LDS column arrays: float (the reference's
 // accumulation, calc_ah_z c2D.cpp:640-751), or double for the FP64-
-// accumulation option, which also leaves out the main-row path (its LDS
-// addressing is float-only) and takes the general row-set path instead.
+// accumulation option (10 MLEM iterations of 64 x 64 x 48, 90 x 96 x 75 took
+// 1.18 ms with its rows on the general row-set path, 1.14 on the folded one;
+// 128^3 10.8 and 10.5, 160^3 21.9 and 21.4).
 template <int S, bool PHASED, class AccT>
 __global__ __launch_bounds__(64 * kBpWaves)
 __attribute__((amdgpu_waves_per_eu(bp_min_waves(S), 8))) void cone_bp_kernel(
@@ -1087,7 +1096,8 @@ __attribute__((amdgpu_waves_per_eu(bp_min_waves(S), 8))) void cone_bp_kernel(
     const float *__restrict__ dpix, float *__restrict__ vol, int acc_in,
     double *__restrict__ norm) {
   constexpr int narr = PHASED ? 1 : S;  // LDS arrays per wavefront
-  constexpr bool kFloatAcc = std::is_same<AccT, float>::value;
+  typedef __attribute__((address_space(3))) AccT lds_acc;
+  constexpr uint32_t kCell = sizeof(AccT);
   extern __shared__ float smem[];
   const int nz = g.nz, nv = g.nv;
   // slice planes, clamped at both ends: s_vz1[q] = plane min(max(q, 0), nz)
@@ -1155,7 +1165,7 @@ __attribute__((amdgpu_waves_per_eu(bp_min_waves(S), 8))) void cone_bp_kernel(
                          one_set && g.bp_main_safe && vb >= min_v && min(vb + span, nv) <= max_v,
                          one_set, min_v, max_v);
       continue;
-    } else if (kFloatAcc && one_set && g.bp_main_safe) {
+    } else if (one_set && g.bp_main_safe) {
       // Every row in one row set (c2D.cpp:657-749): the floor form below
       // min_v (set 0), the truncating form from there on, the second slice
       // below the row's first under the source row g.mid and above it from
@@ -1178,10 +1188,10 @@ __attribute__((amdgpu_waves_per_eu(bp_min_waves(S), 8))) void cone_bp_kernel(
         kb[t] = v < nv ? (floor_form ? g.pzbz1 : g.pzbz) : kBpOff;
         dzv[t] = g.dz[vv];
         izv[t] = g.iz[vv];
-        const uint32_t ks4 = floor_form ? 4u : 0u;
-        b0[t] = lds_addr(reinterpret_cast<const float *>(acc + t * astride + kBpPad)) - ks4;
-        b1[t] = lower ? b0[t] - 4u : b0[t] + 4u;
-        bz[t] = lds_addr(s_vz1) - ks4 + (lower ? 0u : 4u);
+        const uint32_t ks = floor_form ? 1u : 0u;
+        b0[t] = (uint32_t)(uintptr_t)(lds_acc *)(acc + t * astride + kBpPad) - kCell * ks;
+        b1[t] = lower ? b0[t] - kCell : b0[t] + kCell;
+        bz[t] = lds_addr(s_vz1) - 4u * ks + (lower ? 0u : 4u);
       }
       const int khi = nz + 2;
       auto live = [&](const BpRec &rec) {
@@ -1206,20 +1216,24 @@ __attribute__((amdgpu_waves_per_eu(bp_min_waves(S), 8))) void cone_bp_kernel(
         // slice (mz = a1) has c1 = 0 and leaves its second slice alone:
         // adding a zero changes no cell, and the lanes left out of an LDS
         // round take no bank cycles (most segments cross no plane)
-        lds_f32 *c0p[S], *c1p[S];
-        float c0[S], c1[S], o0[S];
+        lds_acc *c0p[S], *c1p[S];
+        float c0[S], c1[S];
+        AccT o0[S];
+        auto cell = [](int k, uint32_t base) {
+          return (lds_acc *)(uintptr_t)cell_add<AccT>(k, base);
+        };
 #pragma unroll
         for (int t = 0; t < S; ++t) {
           const int k = med3_m2s((int)(kb[t] + ai * dzv[t]), khi);
           if constexpr (dir < 0) {
-            c1p[t] = lds_ptr(k4_add(k, b1[t]));
+            c1p[t] = cell(k, b1[t]);
             c0p[t] = c1p[t] + 1;
           } else if constexpr (dir > 0) {
-            c0p[t] = lds_ptr(k4_add(k, b0[t]));
+            c0p[t] = cell(k, b0[t]);
             c1p[t] = c0p[t] + 1;
           } else {
-            c0p[t] = lds_ptr(k4_add(k, b0[t]));
-            c1p[t] = lds_ptr(k4_add(k, b1[t]));
+            c0p[t] = cell(k, b0[t]);
+            c1p[t] = cell(k, b1[t]);
           }
           const float az = *lds_ptr(k4_add(k, bz[t])) * izv[t];
           const float mz = min_sv(a1, az);
