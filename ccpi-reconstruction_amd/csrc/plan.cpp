@@ -288,10 +288,10 @@ size_t Projector::bp_norm_parts() const {
   return cone ? cone_bp_norm_parts(*cone) : par_bp_norm_parts(*par);
 }
 
-void Projector::bp_scaled(const float *dpix, float *vol, hipStream_t st, bool acc_in,
+void Projector::bp_scaled(const float *dpix, float *vol, hipStream_t st, bool f64, bool acc_in,
                           double *norm) const {
   CCPI_REQUIRE(cone, CCPI_E_ARG, "pre-scaled backprojection is a cone-beam form");
-  cone_bp_scaled(*cone, dpix, vol, st, false, acc_in, norm);
+  cone_bp_scaled(*cone, dpix, vol, st, f64, acc_in, norm);
 }
 
 void Projector::bp(const float *sino, float *vol, hipStream_t st, float *scratch, bool f64,

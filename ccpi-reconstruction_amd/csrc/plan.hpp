@@ -279,7 +279,7 @@ struct Projector {
           bool f64 = false, bool acc_in = true, double *norm = nullptr) const;
   // BP of an already scaled sinogram in the padded BP layout (cone only):
   // a solver's fused update kernels write it
-  void bp_scaled(const float *dpix, float *vol, hipStream_t st, bool acc_in = true,
+  void bp_scaled(const float *dpix, float *vol, hipStream_t st, bool f64, bool acc_in = true,
                  double *norm = nullptr) const;
   size_t bp_scratch_floats() const;
   size_t fp_norm_parts() const;
