@@ -132,10 +132,11 @@ __attribute__((amdgpu_waves_per_eu(kParShareWavesPerSimd, 8))) void batch_fp_sha
 // sets, so a batch of one kind gets the kernel of that body alone.
 // Waves per SIMD the registers must allow.  The FP items wait on their
 // gathers: 6 waves took the 64-problem mix from 23.7 to 24.2 CGLS iterations
-// a second.  The tiled BP items: an iteration of the mix takes 30.4 / 28.3 /
-// 28.4 ms with them at 6 / 5 / 4 waves.
+// a second.  The tiled BP items: an iteration of the mix takes 17.4 / 17.7 /
+// 18.2 ms with them at 6 / 5 / 4 waves, one of 8 problems up to 300 columns
+// 0.60 / 0.62 / 0.61.
 template <int MODE, int BPK>
-constexpr int batch_min_waves() { return MODE == 0 ? 6 : BPK == 1 ? 5 : 1; }
+constexpr int batch_min_waves() { return MODE == 0 || BPK == 1 ? 6 : 1; }
 
 template <int RC, int MODE, int BPK>
 __global__ __launch_bounds__(256)

@@ -117,6 +117,7 @@ struct ParArgs {
   double D;              // detector line distance 2 * max|origin|
   double dconv;          // float(3 D) as double: walk start bound
   double ihp, hp0;       // detector column index map
+  int h_even;            // every column lies where the index map puts it (to kEps / 4)
   const double *atab;    // [na][5]: c, s, y_offset, 1/y_offset, length
   const double *h_pix;   // [nh]
   const int *map;        // [nv] row -> slice

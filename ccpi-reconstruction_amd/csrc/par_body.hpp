@@ -36,6 +36,19 @@ __device__ inline float4 load_f4(const CCPI_GLOBAL float *p) {
   return v;
 }
 
+// Minimum and maximum of numbers, without the canonicalisation that the
+// library's take for a signalling NaN.
+__device__ inline double min_f64(double a, double b) {
+  double r;
+  asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ inline double max_f64(double a, double b) {
+  double r;
+  asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
 // LDS byte address of a shared-memory pointer.
 __device__ inline uint32_t lds_byte(const void *p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
@@ -912,18 +925,19 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // one coalesced copy per tile instead of each lane re-reading its columns'
 // rows, and with the columns' positions; every lane then weighs its own
 // column's footprint (the reference's FP64 arithmetic) on the staged rows.
-// Bound by vector issue, about 150 instructions per column and angle of
-// which 60 are the 16 slices' products and sums.  So there are two blocks of
-// LDS and the next one's reads go straight there while this one is summed
-// (one barrier a block, no register in between), spans are found 256 angles
-// at a time, tables are scalar loads, and where no footprint of the
-// wavefront has more than two columns (pixels about as wide as a voxel or
-// wider) both are weighed without a loop.  With the rows staged through
-// registers between two barriers and a loop over positions in global memory
-// it took: 512 x 512 x 32, 360 angles 1.40 ms, now 0.89; 383 x 383 x 29, 180
-// angles 0.44, now 0.31; 256 x 256 x 16, 180 angles 0.116, now 0.081;
-// 64 x 64 x 1, 90 angles 0.027, now 0.021.  32 slices per lane: 0.86 at
-// 512 x 512 x 32 but 0.38 at 383 x 383 x 29.  Angles are visited in order, so with
+// Bound by vector issue (busy all the time at 512 x 512 x 32), about 115
+// instructions per column and angle of which 64 are the 16 slices' products
+// and sums.  So there are two blocks of LDS and the next one's reads go
+// straight there while this one is summed (one barrier a block, no register
+// in between), spans are found 256 angles at a time, tables are scalar loads,
+// and where a voxel's shadow is under two columns wide (pixels about as wide
+// as a voxel or wider) two columns are weighed without a loop, a last column
+// or tests that even columns answer.  With the rows staged through registers
+// between two barriers and a loop over positions in global memory it took:
+// 512 x 512 x 32, 360 angles 1.40 ms, now 0.68; 383 x 383 x 29, 180 angles
+// 0.44, now 0.24; 256 x 256 x 16, 180 angles 0.116, now 0.066; 64 x 64 x 1, 90
+// angles 0.027, now 0.019; with the staging alone 0.89, 0.31, 0.081 and
+// 0.021.  Angles are visited in order, so with
 // one angle group the result is bit-identical to par_bp_kernel; with G
 // groups (blockIdx.z) each group writes its partial sums of its angle range
 // to part[group] and par_bp_sum_kernel adds them in group order.
@@ -942,6 +956,7 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // bit what the grouped launch and par_bp_sum_kernel give into a zeroed
 // volume, without registers for a second set of sums.
 constexpr int kParBpSpans = 256;   // one per thread
+constexpr int kParBpNarrow = 1 << 30;
 template <int R, class Acc, bool FOLD = false>
 __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, int a_end,
                               int hmax, int ab, bool acc_in, const float *__restrict__ sino,
@@ -970,7 +985,6 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
     acc[q] = (!FOLD && acc_in && active && q < nk) ? (Acc)vcol[q] : (Acc)0;
   const double x0 = g.ox + (double)i * g.dx, xn = g.ox + (double)(i + 1) * g.dx;
   const double y0 = g.oy + (double)j * g.dy, yn = g.oy + (double)(j + 1) * g.dy;
-  const double hpix0 = cmem(g.h_pix)[0];
   // rows of the lane's slices that exist (one row per slice)
   const int nrow = max(0, min(R, min(nv, nz) - k0));
 
@@ -992,7 +1006,12 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
     const double tmax = fmax(fmax(p0, p1), fmax(p2, p3));
     const int lo = max((int)floor(tmin * g.ihp - g.hp0) - 2, 0);
     const int hi = min((int)floor(tmax * g.ihp - g.hp0) + 2, nh - 1);
-    s_span[tid] = make_int2(lo, max(0, min(hi - lo + 1, hmax)));
+    // a voxel's shadow under two columns wide, on even columns and a general
+    // line: see the two-column form below
+    const bool narrow = g.h_even != 0 && !(fabs(c) < kEps || fabs(s) < kEps) &&
+                        (fabs(c) * g.dy + fabs(s) * g.dx) * g.ihp < 1.99;
+    s_span[tid] =
+        make_int2(lo, max(0, min(hi - lo + 1, hmax)) | (narrow ? kParBpNarrow : 0));
   };
   // Starts the reads of angles [a0, a0 + n) into buffer `buf`: per wavefront
   // one angle at a time, straight into LDS.  Rows of 16-byte aligned start go
@@ -1004,7 +1023,7 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
     for (int t = wave; t < n; t += 4) {
       const int2 sp = s_span[a0 + t - sb];
       const int lo = __builtin_amdgcn_readfirstlane(sp.x);
-      const int cnt = __builtin_amdgcn_readfirstlane(sp.y);
+      const int cnt = __builtin_amdgcn_readfirstlane(sp.y) & ~kParBpNarrow;
       const int slot = buf * ab + t;
       if (lane == 0) s_cur[slot] = sp;
       const uint32_t row_lds = lds_byte(s_rows + (size_t)slot * hmax * R);
@@ -1053,11 +1072,15 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
       start(next, min(ab, next_gb - next), buf ^ 1, sb);
     }
     if (active) {
+      int2 cur = s_cur[buf * ab];
       for (int t = 0; t < nblk; t++) {
         const CCPI_CONST double *tab = cmem(g.atab) + 5 * (a0 + t);
-        const double c = tab[0], s = tab[1];
+        const double c = tab[0], s = tab[1], t2 = tab[2], t3 = tab[3], l = tab[4];
         const int slot = buf * ab + t;
-        const int slo = s_cur[slot].x, scnt = s_cur[slot].y;
+        const int slo = __builtin_amdgcn_readfirstlane(cur.x);
+        const int sy = __builtin_amdgcn_readfirstlane(cur.y);
+        cur = s_cur[slot + 1];   // the next angle's (the last one's is not used)
+        const int scnt = sy & ~kParBpNarrow;
         const float *rows_t = s_rows + (size_t)slot * hmax * R;
         const double *hp_t = s_hp + (size_t)slot * hmax;
         auto add = [&](const float *pr, float wf) {
@@ -1070,52 +1093,53 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
             acc[4 * q4 + 3] = acc[4 * q4 + 3] + (Acc)(v.w * wf);
           }
         };
-        if (!(fabs(c) < kEps || fabs(s) < kEps)) {
-          // General line: par_footprint and par_weight value for value
-          // (p2D.cpp:881-938).  The footprint's first column lies at or
-          // before ymin, so columns as wide as a voxel's shadow or wider leave
-          // at most two more; both are weighed without a loop when that
-          // holds for the whole wavefront and they are staged.
-          double ymin, ymax;
-          if (c > 0.0) {
-            if (s > 0.0) { ymin = y0 * c - xn * s; ymax = yn * c - x0 * s; }
-            else         { ymin = y0 * c - x0 * s; ymax = yn * c - xn * s; }
-          } else {
-            if (s > 0.0) { ymin = yn * c - xn * s; ymax = y0 * c - x0 * s; }
-            else         { ymin = yn * c - x0 * s; ymax = y0 * c - xn * s; }
-          }
-          const int lo = ymin < hpix0 ? 0 : max((int)floor(ymin * g.ihp - g.hp0), 0);
-          const int hi = min((int)floor(ymax * g.ihp - g.hp0), nh - 1);
-          const int hh = lo - slo;
-          const double e0 = ymin + kEps;
-          bool quick = hh >= 0 && hh + 2 < scnt && hi <= lo + 2;
-          if (quick) quick = !(hp_t[hh] > e0);
-          if (__ballot(!quick) == 0) {
-            const double t2 = tab[2], t3 = tab[3], l = tab[4];
-            const double ybot = ymin + t2, ytop = ymax - t2, e1 = ymax - kEps;
-            const float *pr = rows_t + (hh + 1) * R;
-#pragma unroll
-            for (int u = 1; u <= 2; u++) {
-              const double hp = hp_t[hh + u];
-              const bool rise = hp < ybot, flat = !rise && hp <= ytop;
-              const double d = rise ? hp - ymin : ymax - hp;
-              const double w = flat ? l : l * d * t3;
-              if (lo + u <= hi && hp > e0 && (rise || flat || hp < e1))
-                add(pr + (u - 1) * R, (float)w);
-            }
-            continue;
+        // The two-column form: par_footprint's and par_weight's values
+        // (p2D.cpp:881-938) for the columns lo + 1 and lo + 2, lo the one at
+        // or before ymin.  On even columns lo itself is not hit, a shadow
+        // under two columns wide ends before lo + 3, and the columns past it
+        // fail the weight's own limits, so neither a last column nor a loop
+        // is needed.  The signs of c and s choose which of the products is
+        // which: their minimum and maximum.
+        bool two = false, use1 = false, use2 = false;
+        float w1 = 0.0f, w2 = 0.0f;
+        const float *pr = rows_t;
+        if (sy & kParBpNarrow) {
+          const double yc0 = y0 * c, yc1 = yn * c, xs0 = x0 * s, xs1 = xn * s;
+          const double ymin = min_f64(yc0, yc1) - max_f64(xs0, xs1);
+          const int hh = (int)floor(ymin * g.ihp - g.hp0) - slo;
+          // both staged; a footprint from before the first column goes below
+          two = __builtin_amdgcn_ballot_w64((unsigned)hh >= (unsigned)max(scnt - 2, 0)) == 0;
+          if (two) {
+            const double ymax = max_f64(yc0, yc1) - min_f64(xs0, xs1);
+            const double e0 = ymin + kEps, ybot = ymin + t2, ytop = ymax - t2;
+            const double e1 = max_f64(ymax - kEps, ytop);
+            const float lf = (float)l;
+            auto weigh = [&](double hp, bool &use, float &w) {
+              const double d = min_f64(hp - ymin, ymax - hp);
+              w = hp >= ybot && hp <= ytop ? lf : (float)(l * d * t3);
+              use = hp > e0 && hp < e1;
+            };
+            weigh(hp_t[hh + 1], use1, w1);
+            weigh(hp_t[hh + 2], use2, w2);
+            pr = rows_t + (hh + 1) * R;
           }
         }
-        const ParFoot f = par_footprint(g, tab, x0, xn, y0, yn);
-        for (int h = f.lo; h <= f.hi; h++) {
-          // inside the staged span (see above); the clamp keeps the reads there
-          const int hh = max(min(h - slo, scnt - 1), 0);
-          double w;
-          const int use = par_weight(g, tab, f, hp_t[hh], w);
-          if (use == 0) continue;
-          if (use < 0) break;
-          add(rows_t + (size_t)hh * R, (float)w);
+        if (!two) {
+          const ParFoot f = par_footprint(g, tab, x0, xn, y0, yn);
+          for (int h = f.lo; h <= f.hi; h++) {
+            // inside the staged span (see above); the clamp keeps the reads there
+            const int hh = max(min(h - slo, scnt - 1), 0);
+            double w;
+            const int use = par_weight(g, tab, f, hp_t[hh], w);
+            if (use == 0) continue;
+            if (use < 0) break;
+            add(rows_t + (size_t)hh * R, (float)w);
+          }
         }
+        // after both forms: in one of them alone, the sums would be copied
+        // between two register sets for each angle
+        if (use1) add(pr, w1);
+        if (use2) add(pr + R, w2);
       }
     }
     if (FOLD && group_ends && grp + 1 < ngrp) {

@@ -109,8 +109,8 @@ __global__ __launch_bounds__(256) void par_bp_kernel(ParArgs g,
 // their partial sums to part[group] for par_bp_sum_kernel.  norm (one
 // group only): one partial of ||vol||^2 per workgroup.  5 waves per SIMD
 // (96 VGPRs, a few spills in the set-up): at 4 / 5 / 6 waves the
-// 512 x 512 x 32 BP takes 0.94 / 0.89 / 0.93 ms, 383 x 383 x 29 (ragged)
-// 0.39 / 0.31 / 0.33 and 256 x 256 x 16 0.079 / 0.081 / 0.090.  The
+// 512 x 512 x 32 BP takes 0.72 / 0.68 / 0.66 ms, 383 x 383 x 29 (ragged)
+// 0.31 / 0.24 / 0.24 and 256 x 256 x 16 0.065 / 0.066 / 0.068.  The
 // FP64-accumulation instances keep their registers.
 template <class Acc>
 constexpr int par_bp_lds_min_waves() { return std::is_same<Acc, float>::value ? 5 : 1; }
@@ -262,6 +262,9 @@ static ParTables par_tables(const Geometry &G, ParArgs &A) {
   A.dconv = (double)(float)(3.0 * A.D);
   A.ihp = 1.0 / (G.h_pix[1] - G.h_pix[0]);
   A.hp0 = G.h_pix[0] / (G.h_pix[1] - G.h_pix[0]);
+  A.h_even = 1;
+  for (int h = 0; h < G.nh; h++)
+    if (!(std::fabs(G.h_pix[h] - ((double)h + A.hp0) / A.ihp) < 0.25 * kEps)) A.h_even = 0;
   ParTables T;
   // row -> slice map and its pattern (p2D.cpp:22-61)
   std::vector<int> &map = T.map, &rlo = T.rlo, &rhi = T.rhi;
