@@ -45,6 +45,10 @@ CASES = {
     "starts_inside": PB((40, 40, 16), V1, _turn(60, 0.1), np.arange(30) - 7.3, centred(16, 1.0)),
     "ends_inside": PB((40, 40, 16), V1, _turn(60, 0.1), np.arange(30) - 25.6, centred(16, 1.0)),
     "ragged": PB((17, 49, 13), V1, _turn(45, 0.2), centred(58, 1.0, -0.3), centred(13, 1.0)),
+    "finest_16": PB((17, 18, 12), V1, _turn(20, 0.3), centred(570, 0.0453, 0.01),
+                    centred(12, 1.0)),
+    "finest_8": PB((17, 18, 8), V1, _turn(14, 0.3), centred(1160, 0.0223, 0.01),
+                   centred(8, 1.0)),
     "not_square": PB((24, 40, 16), (1.3, 0.6, 1.0), _turn(60, 0.4), centred(46, 0.9, 0.1),
                      centred(16, 1.0)),
 }
