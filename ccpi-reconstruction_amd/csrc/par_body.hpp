@@ -58,11 +58,11 @@ __device__ inline uint32_t lds_byte(const void *p) {
 // waits for the wavefront's, and a barrier after it shows them to the others.
 __device__ inline void lds_load16(uint32_t lds, const CCPI_GLOBAL float *p) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(p) : "memory");
+               :: "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(p) : "m0", "memory");
 }
 __device__ inline void lds_load4(uint32_t lds, const CCPI_GLOBAL float *p) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off"
-               :: "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(p) : "memory");
+               :: "s"(__builtin_amdgcn_readfirstlane((int)lds)), "v"(p) : "m0", "memory");
 }
 __device__ inline void lds_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
