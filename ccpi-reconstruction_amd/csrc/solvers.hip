@@ -393,20 +393,24 @@ WorkspaceLease::WorkspaceLease() {
 
 WorkspaceLease::~WorkspaceLease() {
   if (!keep_ || w_->bytes() > kKeptBytes) return;
-  KeptWorkspaces &k = kept();
   std::list<std::pair<int, std::unique_ptr<Workspace>>> over;   // freed outside the lock
-  std::lock_guard<std::mutex> lk(k.mu);
-  k.idle.emplace_front(dev_, std::move(w_));
-  size_t n = 0, b = 0;
-  for (auto it = k.idle.begin(); it != k.idle.end();) {
-    const auto q = it++;
-    n++;
-    b += q->second->bytes();
-    if (n > kKeptWorkspaces || b > kKeptBytes) {
-      b -= q->second->bytes();
-      n--;
-      over.splice(over.end(), k.idle, q);
+  try {
+    KeptWorkspaces &k = kept();
+    std::lock_guard<std::mutex> lk(k.mu);
+    k.idle.emplace_front(dev_, std::move(w_));
+    size_t n = 0, b = 0;
+    for (auto it = k.idle.begin(); it != k.idle.end();) {
+      const auto q = it++;
+      n++;
+      b += q->second->bytes();
+      if (n > kKeptWorkspaces || b > kKeptBytes) {
+        b -= q->second->bytes();
+        n--;
+        over.splice(over.end(), k.idle, q);
+      }
     }
+  } catch (...) {
+    // not kept: no host memory for the list, and a destructor does not throw
   }
 }
 
