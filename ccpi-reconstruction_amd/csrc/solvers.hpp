@@ -11,6 +11,7 @@ namespace ccpi {
 // Scalars of one CGLS run, kept in device memory.
 struct CglsScalars {
   double gamma;      // ||A^T r||^2 (FP64 mode)
+  double gamma_next; // the same, of the newest residual (the summing updates)
   float gamma_f;     // same, float mode
   float alpha_f;     // step applied to x and r
   float beta_f;      // direction update factor
