@@ -10,6 +10,7 @@
 #include <string>
 
 #include "ccpi_hip.h"
+#include "grid.hpp"
 
 namespace ccpi {
 
@@ -33,6 +34,19 @@ struct Error : std::runtime_error {
   do {                                                                      \
     if (!(cond)) throw ::ccpi::Error((code), (msg));                        \
   } while (0)
+
+// Number of a workgroup of a wg_grid launch.
+__device__ inline int wg_index() {
+  return (int)(blockIdx.x + (blockIdx.y << kGridRowBits));
+}
+
+// Grid of a wg_grid launch of `blocks` workgroups; `what` names what there
+// are too many of.
+inline dim3 wg_dim3(long long blocks, int threads, const char *what) {
+  const WgGrid G = wg_grid(blocks, threads);
+  CCPI_REQUIRE(G.x != 0, CCPI_E_LIMIT, what);
+  return dim3(G.x, G.y);
+}
 
 // Model tolerance of every branch decision (p2D.cpp:20, c2D.cpp:15).
 constexpr double kEps = 1.1920928955078125e-07;  // FLT_EPSILON

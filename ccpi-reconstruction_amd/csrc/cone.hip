@@ -233,7 +233,6 @@ constexpr int kFpRows = 256;
 // with its own L2.  xcd_block maps the hardware id to a logical id so that
 // every XCD runs one contiguous range of logical ids: neighbouring work
 // (adjacent voxel columns) then shares an L2.
-constexpr int kXcds = 8;
 __device__ inline int xcd_block(int bid, int n) {
   const int xcd = bid % kXcds, local = bid / kXcds;
   const int per = n / kXcds, rem = n % kXcds;
@@ -505,7 +504,7 @@ __global__ __launch_bounds__(kFpRows) void cone_fp_kernel(
   const int nrays = g.na * g.nh;
   // workgroup -> (row block, angle, column) through the XCD's tile
   const int wgs = g.fp_tile_a * kFpTileH;
-  const int xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
+  const int id = wg_index(), xcd = id % kXcds, local = id / kXcds;
   const int tile = (local / wgs) * kXcds + xcd, within = local % wgs;
   const int nth = (g.nh + kFpTileH - 1) / kFpTileH;
   const int nta = (g.na + g.fp_tile_a - 1) / g.fp_tile_a;
@@ -1747,11 +1746,11 @@ static void cone_fp_launch(const ConePlan &P, const float *vol, float *sino, hip
   const long long tiles = (long long)A.fp_blocks * ((A.na + A.fp_tile_a - 1) / A.fp_tile_a) *
                           ((A.nh + kFpTileH - 1) / kFpTileH);
   const long long blocks = (tiles + kXcds - 1) / kXcds * kXcds * (A.fp_tile_a * kFpTileH);
-  CCPI_REQUIRE(blocks < (1LL << 31), CCPI_E_LIMIT, "cone FP: too many rays");
+  const dim3 grid = wg_dim3(blocks, A.fp_threads, "cone FP: too many rays");
   const size_t lds = sizeof(float) * (size_t)(A.nz + 1 + 2 * kFpPad);
-  hipLaunchKernelGGL((cone_fp_kernel<BIG, Acc>), dim3((unsigned)blocks), dim3(A.fp_threads), lds,
-                     st, A, P.rays.as<ConeRay>(), P.ents.as<ConeEnt>(), P.eai.as<float>(), vol,
-                     sino, acc_in ? 1 : 0, norm);
+  hipLaunchKernelGGL((cone_fp_kernel<BIG, Acc>), grid, dim3(A.fp_threads), lds, st, A,
+                     P.rays.as<ConeRay>(), P.ents.as<ConeEnt>(), P.eai.as<float>(), vol, sino,
+                     acc_in ? 1 : 0, norm);
   CCPI_HIP(hipGetLastError());
 }
 
