@@ -521,7 +521,8 @@ constexpr int kParTileA = 32;
 
 // Workgroup `id` -> its rays and rows: ids go to the 8 XCDs in turn, each
 // XCD's in tiles of kParTileA angles of the same 64 columns; row blocks
-// slowest.  index: the workgroup's place among the live ones.
+// slowest.  index: the workgroup's place among the live ones (ids past the
+// last tile are not live).
 struct ParShareItem {
   int a, h0, v0;
   bool live;

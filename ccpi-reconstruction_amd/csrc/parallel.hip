@@ -87,7 +87,7 @@ __attribute__((amdgpu_waves_per_eu(par_fp_min_waves<Acc>(), 8))) void par_fp_sha
     ParArgs g, int lr, const float *__restrict__ vol, float *__restrict__ sino, int acc_in,
     double *__restrict__ norm) {
   __shared__ ParShare sh;
-  const ParShareItem it = par_share_item(g, lr, blockIdx.x);
+  const ParShareItem it = par_share_item(g, lr, wg_index());
   if (!it.live) return;
   const double ss = par_fp_shared<NS, VEC, Acc>(g, it.a, it.h0, it.v0, lr, vol, sino,
                                                 acc_in != 0, sh);
@@ -476,9 +476,7 @@ static ParFpLaunch par_fp_launch_of(const ParArgs &A) {
   if (L.form == ParFpForm::kShared) {
     L.n = std::min(L.lr, 2);
     L.threads = 64 * (1 + L.lr / L.n);
-    const long long items = par_share_items(A, L.lr);
-    CCPI_REQUIRE(items < (1LL << 31), CCPI_E_LIMIT, "parallel FP: too many rays");
-    L.grid = dim3((unsigned)items);
+    L.grid = wg_dim3(par_share_items(A, L.lr), L.threads, "parallel FP: too many rays");
     L.parts = par_share_parts(A, L.lr);
     return L;
   }

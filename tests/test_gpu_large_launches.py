@@ -47,3 +47,15 @@ def test_cone_fp_of_2_32_pixels():
                           source=(-40.0, 0.0, 0.0), detector_x=40.0)
     x = torch.rand(8, 8, 16, generator=torch.Generator().manual_seed(3)).cuda() + 0.1
     _check(geom, x)
+
+
+def test_parallel_fp_of_2_32_threads():
+    # 64 rays a workgroup of 576 threads: two columns fill it least
+    na, nh, nv = 7_460_001, 2, 33
+    ang = np.linspace(0, np.pi, na, endpoint=False) + 0.01
+    h, v = centred(nh, 1.0, 0.1), centred(nv, 1.0)
+    print(f"\nparallel FP {na} x {nh} x {nv}", flush=True)
+
+    def geom(part):
+        return J.Geometry(ang[part], h, v, (-1, -1, -nv / 2), (1, 1, 1), (2, 2, nv))
+    _check(geom, torch.rand(2, 2, nv, generator=torch.Generator().manual_seed(4)).cuda() + 0.1)
