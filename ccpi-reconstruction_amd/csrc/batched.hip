@@ -97,11 +97,13 @@ __global__ __launch_bounds__(kBatchShareThreads)
 __attribute__((amdgpu_waves_per_eu(kParShareWavesPerSimd, 8))) void batch_fp_shared_kernel(
     const BatchProb *__restrict__ P, BatchLists L) {
   __shared__ ParShare sh;
-  const int p = find_prob(L.fs_off, L.count, blockIdx.x);
+  const int id = wg_index();
+  if (id >= L.fs_off[L.count]) return;
+  const int p = find_prob(L.fs_off, L.count, id);
   const BatchProb &B = P[p];
   const ParArgs g = B.g;
   const int lr = B.fp_lr;
-  const ParShareItem it = par_share_item(g, lr, (int)blockIdx.x - L.fs_off[p]);
+  const ParShareItem it = par_share_item(g, lr, id - L.fs_off[p]);
   if (!it.live) return;
   const float *d = B.d;
   float *Ad = B.Ad;
@@ -344,7 +346,8 @@ struct BatchRun {
 void proj(const BatchRun &R, const Tuned &T, int mode, hipStream_t st) {
   BatchProb *P = R.W.probs.as<BatchProb>();
   if (mode == 0 && R.fs_total > 0) {
-    hipLaunchKernelGGL(batch_fp_shared_kernel, dim3((unsigned)R.fs_total),
+    hipLaunchKernelGGL(batch_fp_shared_kernel,
+                       wg_dim3(R.fs_total, kBatchShareThreads, "batched CGLS: too many rays"),
                        dim3(kBatchShareThreads), 0, st, P, R.L);
     CCPI_HIP(hipGetLastError());
   }

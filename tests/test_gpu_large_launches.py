@@ -4,7 +4,8 @@ HIP takes fewer than 2^32 threads along one grid dimension.  The cases are
 projections whose workgroups times threads pass that, at the smallest data
 that get there.  The rays of one angle do not depend on the other angles, so
 the first, middle and last angles have to equal, bit for bit, the projection
-of a geometry of those angles alone.
+of a geometry of those angles alone; the problems of a batch are checked
+against the one-problem CGLS, within the tolerances of the other batched tests.
 """
 
 import numpy as np
@@ -59,3 +60,24 @@ def test_parallel_fp_of_2_32_threads():
     def geom(part):
         return J.Geometry(ang[part], h, v, (-1, -1, -nv / 2), (1, 1, 1), (2, 2, nv))
     _check(geom, torch.rand(2, 2, nv, generator=torch.Generator().manual_seed(4)).cuda() + 0.1)
+
+
+def test_batch_of_2_32_fp_threads():
+    # 64 rays and 32 rows a workgroup of 320 threads; the two-columns problems
+    # of 33 rows fill them least
+    na, nh, nv, count = 105_001, 2, 33, 64
+    print(f"\nbatched CGLS {count} x {na} x {nh} x {nv}", flush=True)
+    geoms, bs = [], []
+    for q in range(count):
+        ang = np.linspace(0, np.pi, na, endpoint=False) + 0.001 * (q + 1)
+        geoms.append(J.Geometry(ang, centred(nh, 1.0, 0.1), centred(nv, 1.0),
+                                (-1, -1, -nv / 2), (1, 1, 1), (2, 2, nv)))
+        x = torch.rand(2, 2, nv, generator=torch.Generator().manual_seed(q)).cuda() + 0.1
+        bs.append(J.forward_project(geoms[-1], x))
+    xs, rs, norms = J.cgls_batched(geoms, bs, 1)
+    for q in (0, 31, count - 1):
+        x, r, n = J.cgls(geoms[q], bs[q], 1)
+        assert float(x.abs().max()) > 0
+        assert float((xs[q] - x).abs().max()) < 1e-5 * float(x.abs().max())
+        assert float((rs[q] - r).abs().max()) < 1e-5 * float(bs[q].abs().max())
+        assert np.allclose(norms[q], n, rtol=1e-6)
