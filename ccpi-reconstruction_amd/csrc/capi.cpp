@@ -327,6 +327,17 @@ int ccpi_cone_bp_layout(const ccpi_geometry *g, int *row_stride, int *phased, in
   });
 }
 
+int ccpi_cone_bp_rows(const ccpi_geometry *g, int *rows_per_lane, int *phases) {
+  return guarded([&] {
+    CCPI_REQUIRE(rows_per_lane && phases, CCPI_E_ARG, "null output");
+    const ccpi::Geometry G = ccpi::Geometry::from(g);
+    CCPI_REQUIRE(G.kind == CCPI_CONE, CCPI_E_ARG, "BP rows query takes a cone geometry");
+    const ccpi::BpLayout L = ccpi::cone_bp_layout(G);
+    *rows_per_lane = L.rows;
+    *phases = L.row_phases;
+  });
+}
+
 const char *ccpi_error_string(int status) {
   switch (status) {
     case CCPI_OK: return "ok";

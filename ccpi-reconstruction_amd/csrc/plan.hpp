@@ -206,13 +206,13 @@ long long plan_cache_bytes();
 
 // Accumulation layout of the cone BP for a geometry (host only): row stride
 // S (rows per lane at most), whether it is the phased one-array form and its
-// lane phases for that S, the bound
-// on detector rows per slice it was chosen for, the padded row length, and
-// the rows per slice at walk parameter 1 (voxel z size / smallest pitch).
+// lane phases for that S, the bound on detector rows per slice it was chosen
+// for, the padded row length, the rows per slice at walk parameter 1 (voxel z
+// size / smallest pitch), and the rows per lane and lane phases that run.
 struct BpLayout {
   int stride = 1, unique = 1, main_safe = 0, phased = 0, phases = 1, nvp = 0, want = 1;
   double rps1 = 1.0;
-  int rows = 1, row_phases = 1;   // the phased form's rows per lane and lane phases
+  int rows = 1, row_phases = 1;
 };
 BpLayout cone_bp_layout(const Geometry &g);
 

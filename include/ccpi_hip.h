@@ -205,15 +205,20 @@ int ccpi_pb_cgls_batched(const ccpi_geometry *geoms, int count,
 
 /* BP accumulation layout the library picks for a cone geometry, computed
    on the host only (no device work, usable without a GPU): *row_stride =
-   detector rows per lane (S), *phased = 1 for the one-array form whose
-   lanes update in *phases rounds (with fewer rows per lane in as many more
-   rounds for a detector of fewer than 64 * S rows), *rows_bound = the bound on detector rows
-   per voxel slice over all columns that the choice guarantees (lanes of one
-   round are >= that many rows apart, or alone in their round).  No
-   counterpart in the reference: its b2D accumulates each voxel column on
-   one host thread (c2D.cpp:1016-1046). */
+   the most detector rows a lane takes (S), *phased = 1 for the one-array
+   form, whose lanes of S rows each would update in *phases rounds,
+   *rows_bound = the bound on detector rows per voxel slice over all columns
+   that the choice guarantees (lanes of one round are >= that many rows apart,
+   or alone in their round).  The phased form runs with fewer rows per lane
+   and more rounds on a detector that 64 * S rows would not fill:
+   ccpi_cone_bp_rows.  No counterpart in the reference: its b2D accumulates
+   each voxel column on one host thread (c2D.cpp:1016-1046). */
 int ccpi_cone_bp_layout(const ccpi_geometry *g, int *row_stride, int *phased,
                         int *phases, int *rows_bound);
+/* The rows per lane and the rounds that the cone BP of a geometry runs with,
+   within that layout (a voxel column far from the source may run fewer
+   rounds).  Host only, as above. */
+int ccpi_cone_bp_rows(const ccpi_geometry *g, int *rows_per_lane, int *phases);
 
 /* ---- utilities --------------------------------------------------------- */
 const char *ccpi_error_string(int status);
