@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "kept.hpp"
 
 namespace ccpi {
 
@@ -46,10 +47,11 @@ struct Geometry {
   size_t n_pix() const { return (size_t)na * nh * nv; }
 };
 
-// Owning device allocation.
 // Frees the workspaces that calls have left for the next (solvers.hip).
 void workspaces_give_back();
 
+// Owning device allocation.  Where the device is out of memory the idle
+// workspaces go back and it is tried once more.
 struct DeviceBuffer {
   void *p = nullptr;
   size_t bytes = 0;
@@ -65,12 +67,15 @@ struct DeviceBuffer {
   void alloc(size_t n) {
     if (n <= bytes && p) return;
     reset();
-    if (hipMalloc(&p, n ? n : 4) != hipSuccess) {
-      (void)hipGetLastError();
-      p = nullptr;
-      workspaces_give_back();
-      CCPI_HIP(hipMalloc(&p, n ? n : 4));
-    }
+    auto get = [&] {
+      const hipError_t e = hipMalloc(&p, n ? n : 4);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+      }
+      return e;
+    };
+    CCPI_HIP(alloc_giving_back(hipErrorOutOfMemory, get, workspaces_give_back));
     bytes = n;
   }
   template <class T>

@@ -15,9 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <list>
 #include <memory>
-#include <mutex>
 #include <vector>
 
 #include "common.hpp"
@@ -407,61 +405,22 @@ size_t Workspace::bytes() const {
   return b;
 }
 
-namespace {
-struct KeptWorkspaces {
-  std::mutex mu;
-  std::list<std::pair<int, std::unique_ptr<Workspace>>> idle;   // (device, workspace), last left first
-};
-KeptWorkspaces &kept() {
-  static KeptWorkspaces k;
+static Kept<Workspace> &kept() {
+  static Kept<Workspace> k(kKeptWorkspaces, kKeptBytes);
   return k;
 }
-}  // namespace
 
 WorkspaceLease::WorkspaceLease() {
   CCPI_HIP(hipGetDevice(&dev_));
-  KeptWorkspaces &k = kept();
-  {
-    std::lock_guard<std::mutex> lk(k.mu);
-    for (auto it = k.idle.begin(); it != k.idle.end(); ++it)
-      if (it->first == dev_) {
-        w_ = std::move(it->second);
-        k.idle.erase(it);
-        return;
-      }
-  }
-  w_ = std::make_unique<Workspace>();
+  w_ = kept().take(dev_);
+  if (!w_) w_ = std::make_unique<Workspace>();
 }
 
 WorkspaceLease::~WorkspaceLease() {
-  if (!keep_ || w_->bytes() > kKeptBytes) return;
-  std::list<std::pair<int, std::unique_ptr<Workspace>>> over;   // freed outside the lock
-  try {
-    KeptWorkspaces &k = kept();
-    std::lock_guard<std::mutex> lk(k.mu);
-    k.idle.emplace_front(dev_, std::move(w_));
-    size_t n = 0, b = 0;
-    for (auto it = k.idle.begin(); it != k.idle.end();) {
-      const auto q = it++;
-      n++;
-      b += q->second->bytes();
-      if (n > kKeptWorkspaces || b > kKeptBytes) {
-        b -= q->second->bytes();
-        n--;
-        over.splice(over.end(), k.idle, q);
-      }
-    }
-  } catch (...) {
-    // not kept: no host memory for the list, and a destructor does not throw
-  }
+  if (keep_) kept().leave(dev_, std::move(w_));
 }
 
-void workspaces_give_back() {
-  std::list<std::pair<int, std::unique_ptr<Workspace>>> all;
-  KeptWorkspaces &k = kept();
-  std::lock_guard<std::mutex> lk(k.mu);
-  all.swap(k.idle);
-}
+void workspaces_give_back() { kept().give_back(); }
 
 void Workspace::ensure(const Projector &P) {
   const size_t nvox = P.geometry().n_vox(), npix = P.geometry().n_pix();

@@ -1,11 +1,16 @@
 // CPU checks of the library's host rules (csrc headers without HIP types).
 // host_rules <check> exits 0 where the check holds; test_host_rules.py builds
 // and runs it.
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <initializer_list>
+#include <memory>
+#include <thread>
+#include <vector>
 
 #include "grid.hpp"
+#include "kept.hpp"
 
 static int failed = 0;
 #define EXPECT(c) \
@@ -35,9 +40,111 @@ static void grids() {
   }
 }
 
+struct Thing {
+  static std::atomic<int> live;
+  int id;
+  size_t size;
+  std::atomic<int> holders{0};
+  Thing(int i, size_t s) : id(i), size(s) { live++; }
+  ~Thing() { live--; }
+  size_t bytes() const { return size; }
+};
+std::atomic<int> Thing::live{0};
+using Things = ccpi::Kept<Thing>;
+static std::unique_ptr<Thing> thing(int id, size_t size) {
+  return std::make_unique<Thing>(id, size);
+}
+
+// At most 4 and 100 bytes stay, the ones left last; each device its own.
+static void kept() {
+  Things k(4, 100);
+  EXPECT(!k.take(0));
+  for (int i = 0; i < 7; i++) {
+    k.leave(0, thing(i, 10));
+    EXPECT(Thing::live == (i < 4 ? i + 1 : 4));
+  }
+  EXPECT(!k.take(1));
+  for (int i = 6; i >= 3; i--) {
+    auto t = k.take(0);
+    EXPECT(t && t->id == i);
+  }
+  EXPECT(!k.take(0) && Thing::live == 0);
+  // over the bytes together: the older ones go, a small older one may stay
+  k.leave(0, thing(0, 20));
+  k.leave(0, thing(1, 60));
+  k.leave(1, thing(2, 50));
+  EXPECT(Thing::live == 2);
+  auto a = k.take(0);
+  EXPECT(a && a->id == 0);
+  auto b = k.take(1);
+  EXPECT(b && b->id == 2);
+  // one larger than the limit never stays, one of the limit does, alone
+  k.leave(0, std::move(a));
+  k.leave(0, thing(3, 101));
+  EXPECT(Thing::live == 2);
+  k.leave(0, thing(4, 100));
+  EXPECT(Thing::live == 2);   // 4 and the held b
+  k.leave(1, std::move(b));
+  EXPECT(Thing::live == 1);
+  k.give_back();
+  EXPECT(Thing::live == 0 && !k.take(0) && !k.take(1));
+}
+
+// No object has two holders, and no more than the limit stay.
+static void kept_threads() {
+  Things k(4, 1000);
+  std::atomic<bool> shared{false};
+  std::vector<std::thread> ts;
+  for (int n = 0; n < 8; n++)
+    ts.emplace_back([&, n] {
+      for (int i = 0; i < 2000; i++) {
+        auto t = k.take(i % 2);
+        if (!t) t = thing(n, 10 + n);
+        if (t->holders++ != 0) shared = true;
+        std::this_thread::yield();
+        t->holders--;
+        k.leave(i % 2, std::move(t));
+        if (i % 500 == 499) k.give_back();
+      }
+    });
+  for (auto &t : ts) t.join();
+  EXPECT(!shared && Thing::live <= 4);
+  k.give_back();
+  EXPECT(Thing::live == 0);
+}
+
+// A refused allocation is tried once more, after what idles has gone back;
+// another error is not.
+static void refused_allocation() {
+  enum Status { kOk, kRefused, kOther };
+  Things k(4, 1000);
+  auto fill = [&] {
+    for (int i = 0; i < 3; i++) k.leave(0, thing(i, 10));
+  };
+  int tries = 0;
+  auto back = [&] { k.give_back(); };
+  auto room = [&] {
+    tries++;
+    return Thing::live == 0 ? kOk : kRefused;
+  };
+  fill();
+  EXPECT(ccpi::alloc_giving_back(kRefused, room, back) == kOk && tries == 2);
+  EXPECT(ccpi::alloc_giving_back(kRefused, room, back) == kOk && tries == 3);
+  fill();
+  auto held = k.take(0);
+  EXPECT(ccpi::alloc_giving_back(kRefused, room, back) == kRefused && tries == 5);
+  EXPECT(Thing::live == 1);   // the held one is not touched
+  fill();
+  EXPECT(ccpi::alloc_giving_back(kRefused, [] { return kOther; }, back) == kOther);
+  EXPECT(Thing::live == 4);
+}
+
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "grids")) grids();
+  else if (!std::strcmp(what, "kept")) kept();
+  else if (!std::strcmp(what, "kept_threads")) kept_threads();
+  else if (!std::strcmp(what, "refused_allocation")) refused_allocation();
   else return 2;
   return failed;
 }
