@@ -30,7 +30,7 @@ EXPORTS = (
     "ccpi_pb_cgls_batched", "ccpi_cgls_create", "ccpi_cgls_iterate", "ccpi_cgls_norms", "ccpi_cgls_timings",
     "ccpi_cgls_destroy", "ccpi_projector_nnz", "ccpi_cone_bp_layout",
     "ccpi_cone_bp_rows", "ccpi_error_string", "ccpi_last_error", "ccpi_version",
-    "ccpi_plan_cache_clear", "ccpi_plan_cache_bytes",
+    "ccpi_plan_cache_clear", "ccpi_plan_cache_bytes", "ccpi_workspaces_clear",
 )
 
 
@@ -110,6 +110,7 @@ def lib():
     L.ccpi_last_error.restype = C.c_char_p
     L.ccpi_version.restype = C.c_int
     L.ccpi_plan_cache_clear.restype = None
+    L.ccpi_workspaces_clear.restype = None
     L.ccpi_plan_cache_bytes.restype = C.c_longlong
     _lib = L
     return L

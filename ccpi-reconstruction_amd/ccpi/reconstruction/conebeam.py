@@ -50,10 +50,11 @@ def _reconstruct(algo, pixels, angles, h_offsets, v_offsets, pixels_per_voxel,
     dx = float(source_to_detector) + sx
     setup = _ins.xtek_setup(pix.shape, angles, int(pixels_per_voxel), sx, dx,
                             float(pixel_h_size), float(pixel_v_size), float(mask_radius))
-    b = _ins.xtek_read_scans(torch.from_numpy(pix).to(dev), setup, bool(is_pixels_in_log))
+    b = _pj.with_room(lambda: _ins.xtek_read_scans(torch.from_numpy(pix).to(dev), setup,
+                                                   bool(is_pixels_in_log)))
     g = setup.geometry
     _ins.find_centre(setup, b, g.v_pixels.size // 2)
-    x = torch.zeros(g.shape, dtype=torch.float32, device=dev)
+    x = _pj.with_room(lambda: torch.zeros(g.shape, dtype=torch.float32, device=dev))
     if algo == "cgls":
         x, _, norms = _pj.cgls(g, b, int(niterations), x)
         _last["norms"] = norms

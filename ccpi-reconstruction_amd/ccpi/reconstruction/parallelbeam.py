@@ -63,8 +63,9 @@ def _reconstruct(pixels, angles, rotation_centre, resolution, niterations, is_lo
         raise ValueError("pixels must be [angle][v][h]")
     setup = _ins.diamond_setup(pix.shape, angles, float(rotation_centre), int(resolution))
     g = setup.geometry
-    b = _ins.diamond_read_scans(torch.from_numpy(pix).to(dev), setup, bool(is_log))
-    x = torch.zeros(g.shape, dtype=torch.float32, device=dev)
+    b = _pj.with_room(lambda: _ins.diamond_read_scans(torch.from_numpy(pix).to(dev), setup,
+                                                      bool(is_log)))
+    x = _pj.with_room(lambda: torch.zeros(g.shape, dtype=torch.float32, device=dev))
     if x0 is not None:
         x0 = _as_f32(x0, "last_iteration_volume")
         if x0.shape != g.shape:

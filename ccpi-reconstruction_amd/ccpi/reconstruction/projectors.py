@@ -92,13 +92,40 @@ def _dev(t, shape, name):
     return C.c_void_p(t.data_ptr())
 
 
+def with_room(make):
+    """``make()``, which allocates device memory of torch's.  Where the device
+    has none left, once more after the kept workspaces have gone back, which
+    torch's allocator does not know of.  (Plans stay: a captured graph may
+    read their tables.)"""
+    import torch
+    try:
+        return make()
+    except torch.cuda.OutOfMemoryError:
+        pass
+    workspaces_clear()
+    return make()
+
+
+def _zeros(shape, device):
+    import torch
+    return with_room(lambda: torch.zeros(shape, dtype=torch.float32, device=device))
+
+
+def _empty(shape, device):
+    import torch
+    return with_room(lambda: torch.empty(shape, dtype=torch.float32, device=device))
+
+
+def _copy(b):
+    return with_room(lambda: b.detach().clone().contiguous())
+
+
 def forward_project(geom: Geometry, vol, out=None):
     """Sinogram of ``vol``.  With ``out`` given the projection accumulates
     into it (parallel) or into it and then scales by d_conv (cone), as
     f2D does (p2D.cpp:468-611, c2D.cpp:469-625)."""
-    import torch
     if out is None:
-        out = torch.zeros(geom.sino_shape, dtype=torch.float32, device=vol.device)
+        out = _zeros(geom.sino_shape, vol.device)
     pv = _dev(vol, geom.shape, "vol")
     po = _dev(out, geom.sino_shape, "out")
     check(lib().ccpi_forward_project(C.byref(geom.c_struct()), po, pv, _stream()))
@@ -108,9 +135,8 @@ def forward_project(geom: Geometry, vol, out=None):
 def backward_project(geom: Geometry, sino, out=None):
     """Backprojection of ``sino``, accumulated into ``out`` if given
     (p2D.cpp:950-1087, c2D.cpp:948-1119)."""
-    import torch
     if out is None:
-        out = torch.zeros(geom.shape, dtype=torch.float32, device=sino.device)
+        out = _zeros(geom.shape, sino.device)
     ps = _dev(sino, geom.sino_shape, "sino")
     po = _dev(out, geom.shape, "out")
     check(lib().ccpi_backward_project(C.byref(geom.c_struct()), ps, po, _stream()))
@@ -121,10 +147,9 @@ def cgls(geom: Geometry, b, iterations: int, x=None, reduce_fp32: bool = False):
     """CGLS body (cgls.cpp:26-157).  Returns (x, residual, norms) where the
     residual is b - A x and norms[i] = ||A^T r|| after iteration i.  ``b``
     is not modified (a copy carries the residual)."""
-    import torch
-    r = b.detach().clone().contiguous()
+    r = _copy(b)
     if x is None:
-        x = torch.zeros(geom.shape, dtype=torch.float32, device=b.device)
+        x = _zeros(geom.shape, b.device)
     norms = np.zeros(max(iterations, 1), np.float64)
     check(lib().ccpi_cgls(C.byref(geom.c_struct()), _dev(r, geom.sino_shape, "b"),
                           _dev(x, geom.shape, "x"), int(iterations),
@@ -140,12 +165,11 @@ def regularize(kind: int, vol, out=None):
     """Tikhonov (``TIKHONOV``, tikhonov.cpp:4-32) or TV (``TV``,
     total_v.cpp:21-195) term of a [nx][ny][nz] float32 device volume; every
     extent must be >= 2."""
-    import torch
     if vol.dim() != 3:
         raise ValueError("vol must be [nx][ny][nz]")
     shape = tuple(vol.shape)
     if out is None:
-        out = torch.empty(shape, dtype=torch.float32, device=vol.device)
+        out = _empty(shape, vol.device)
     check(lib().ccpi_regularize(int(kind), _dev(vol, shape, "vol"), _dev(out, shape, "out"),
                                 shape[0], shape[1], shape[2], _stream()))
     return out
@@ -155,10 +179,9 @@ def cgls_reg(geom: Geometry, b, iterations: int, kind: int, lam: float, x=None,
              reduce_fp32: bool = False):
     """Regularised CGLS, cgls_tikhonov / cgls_tv_reg (cgls.cpp:343-435).
     Returns (x, residual, norms) like :func:`cgls`; ``b`` is not modified."""
-    import torch
-    r = b.detach().clone().contiguous()
+    r = _copy(b)
     if x is None:
-        x = torch.zeros(geom.shape, dtype=torch.float32, device=b.device)
+        x = _zeros(geom.shape, b.device)
     norms = np.zeros(max(iterations, 1), np.float64)
     check(lib().ccpi_cgls_reg(C.byref(geom.c_struct()), _dev(r, geom.sino_shape, "b"),
                               _dev(x, geom.shape, "x"), int(iterations), int(kind),
@@ -169,9 +192,8 @@ def cgls_reg(geom: Geometry, b, iterations: int, kind: int, lam: float, x=None,
 
 def sirt(geom: Geometry, b, iterations: int, x=None):
     """SIRT body (sirt.cpp:15-80), starting from ``x`` (zeros if None)."""
-    import torch
     if x is None:
-        x = torch.zeros(geom.shape, dtype=torch.float32, device=b.device)
+        x = _zeros(geom.shape, b.device)
     check(lib().ccpi_sirt(C.byref(geom.c_struct()), _dev(b, geom.sino_shape, "b"),
                           _dev(x, geom.shape, "x"), int(iterations), 0, _stream()))
     return x
@@ -181,9 +203,8 @@ def mlem(geom: Geometry, b, iterations: int, x=None, accum_fp64: bool = False):
     """MLEM body (mlem.cpp:15-80); x is reset to ones first.  With
     ``accum_fp64`` the projections' sums (A x, A^T (b / A x), A^T 1) are
     accumulated in double (C ABI flag CCPI_ACCUM_FP64)."""
-    import torch
     if x is None:
-        x = torch.empty(geom.shape, dtype=torch.float32, device=b.device)
+        x = _empty(geom.shape, b.device)
     check(lib().ccpi_mlem(C.byref(geom.c_struct()), _dev(b, geom.sino_shape, "b"),
                           _dev(x, geom.shape, "x"), int(iterations),
                           CCPI_ACCUM_FP64 if accum_fp64 else 0, _stream()))
@@ -194,12 +215,10 @@ def cgls_batched(geoms: Sequence[Geometry], bs, iterations: int, xs=None,
                  reduce_fp32: bool = False):
     """Independent parallel-beam CGLS problems of uneven sizes in one call.
     Returns (xs, residuals, norms[count][iterations])."""
-    import torch
     n = len(geoms)
-    rs = [b.detach().clone().contiguous() for b in bs]
+    rs = [_copy(b) for b in bs]
     if xs is None:
-        xs = [torch.zeros(g.shape, dtype=torch.float32, device=b.device)
-              for g, b in zip(geoms, bs)]
+        xs = [_zeros(g.shape, b.device) for g, b in zip(geoms, bs)]
     arr = (CcpiGeometry * n)(*[g.c_struct() for g in geoms])
     pb = (C.c_void_p * n)(*[_dev(r, g.sino_shape, "b").value for r, g in zip(rs, geoms)])
     px = (C.c_void_p * n)(*[_dev(x, g.shape, "x").value for x, g in zip(xs, geoms)])
@@ -262,7 +281,15 @@ def projector_nnz(geom: Geometry) -> int:
     return int(n.value)
 
 
+def workspaces_clear() -> None:
+    """Gives back the device memory that solver calls have left for the next
+    one: at most four workspaces, 2 GiB together.  An allocation of torch's
+    outside this package does not do that by itself."""
+    lib().ccpi_workspaces_clear()
+
+
 def plan_cache_clear() -> None:
+    """Drops the cached plans and gives back the kept workspaces."""
     lib().ccpi_plan_cache_clear()
 
 

@@ -356,6 +356,8 @@ int ccpi_version(void) { return 100; }
 
 void ccpi_plan_cache_clear(void) { ccpi::plan_cache_clear(); }
 
+void ccpi_workspaces_clear(void) { ccpi::workspaces_give_back(); }
+
 long long ccpi_plan_cache_bytes(void) { return ccpi::plan_cache_bytes(); }
 
 }  // extern "C"

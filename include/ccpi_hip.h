@@ -227,9 +227,14 @@ const char *ccpi_error_string(int status);
 const char *ccpi_last_error(void);
 int ccpi_version(void);
 /* Drop cached per-geometry plans (device tables) on the current device, and
-   the workspaces that solver calls have left for the next one (at most four,
-   2 GiB together, not counted by ccpi_plan_cache_bytes). */
+   the kept workspaces. */
 void ccpi_plan_cache_clear(void);
+/* Give back the workspaces that solver calls have left for the next one: at
+   most four, 2 GiB together, not counted by ccpi_plan_cache_bytes.  They stay
+   until this call or ccpi_plan_cache_clear, or until an allocation of this
+   library finds the device out of memory; one of another allocator's in the
+   same process that fails does not give them back. */
+void ccpi_workspaces_clear(void);
 /* Device bytes held by cached plans on the current device. */
 long long ccpi_plan_cache_bytes(void);
 
