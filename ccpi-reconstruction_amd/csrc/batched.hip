@@ -20,7 +20,7 @@
 // re-reads Ad or s.  The BP's rows per lane and grid (one workgroup per
 // item, or a persistent grid of 2 / 4 / 8 workgroups per CU dealing the items
 // out by a fixed stride) are picked by timing candidates on the batch itself
-// (autotune, cached per batch shape), and so is the grid of the FP items that
+// (tune_batch, cached per batch shape), and so is the grid of the FP items that
 // the shared walk does not take.
 #include <hip/hip_runtime.h>
 
@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "batch_tune.hpp"
 #include "par_body.hpp"
 #include "plan.hpp"
 #include "solvers.hpp"
@@ -261,17 +262,6 @@ __global__ __launch_bounds__(256) void batch_vec_kernel(BatchProb *__restrict__ 
 
 namespace {
 
-// Launch shape of a batch: slices per BP item (rc) and the grids of the FP
-// items outside the shared walk and of the BP: 0 launches one wavefront per
-// FP item and one workgroup per BP item (the dispatcher balances the uneven items), a
-// positive value is a persistent grid of that many workgroups (capped at
-// residency) that deals the items out by a fixed stride.
-struct Tuned {
-  int rc;
-  int fp_grid;
-  int bp_grid;
-};
-
 std::mutex g_tune_mu;
 std::map<std::string, Tuned> g_tuned;
 
@@ -317,11 +307,9 @@ void launch_bp(int bpk, int grid, int items, size_t lds, BatchProb *P, const Bat
 }
 
 template <int RC>
-void launch_proj(int mode, int bpk, int grid, int items, size_t lds, BatchProb *P,
-                 const BatchLists &L, hipStream_t st) {
-  if (mode == 0)
-    launch_one<RC, 0, 3>(grid, items, lds, P, L, st);  // the FP has no BP body
-  else if (mode == 1)
+void launch_bp_mode(int mode, int bpk, int grid, int items, size_t lds, BatchProb *P,
+                    const BatchLists &L, hipStream_t st) {
+  if (mode == 1)
     launch_bp<RC, 1>(bpk, grid, items, lds, P, L, st);
   else
     launch_bp<RC, 2>(bpk, grid, items, lds, P, L, st);
@@ -343,21 +331,29 @@ struct BatchRun {
   int bp_kinds = 0;    // BP bodies of the problems: 1 tiled, 2 column-per-lane
 };
 
+// FP items outside the shared walk (they have neither BP body nor slices per
+// item: one instance).
+void proj_fp_items(const BatchRun &R, int grid, hipStream_t st) {
+  launch_one<8, 0, 3>(grid, R.fp_total, R.bp_lds, R.W.probs.as<BatchProb>(), R.L, st);
+  CCPI_HIP(hipGetLastError());
+}
+
 void proj(const BatchRun &R, const Tuned &T, int mode, hipStream_t st) {
   BatchProb *P = R.W.probs.as<BatchProb>();
-  if (mode == 0 && R.fs_total > 0) {
-    hipLaunchKernelGGL(batch_fp_shared_kernel,
-                       wg_dim3(R.fs_total, kBatchShareThreads, "batched CGLS: too many rays"),
-                       dim3(kBatchShareThreads), 0, st, P, R.L);
-    CCPI_HIP(hipGetLastError());
+  if (mode == 0) {
+    if (R.fs_total > 0) {
+      hipLaunchKernelGGL(batch_fp_shared_kernel,
+                         wg_dim3(R.fs_total, kBatchShareThreads, "batched CGLS: too many rays"),
+                         dim3(kBatchShareThreads), 0, st, P, R.L);
+      CCPI_HIP(hipGetLastError());
+    }
+    if (R.fp_total > 0) proj_fp_items(R, T.fp_grid, st);
+    return;
   }
-  if (mode == 0 && R.fp_total == 0) return;
-  const int grid = mode == 0 ? T.fp_grid : T.bp_grid;
-  const int items = mode == 0 ? R.fp_total : R.bp_total;
   if (T.rc == 8)
-    launch_proj<8>(mode, R.bp_kinds, grid, items, R.bp_lds, P, R.L, st);
+    launch_bp_mode<8>(mode, R.bp_kinds, T.bp_grid, R.bp_total, R.bp_lds, P, R.L, st);
   else
-    launch_proj<16>(mode, R.bp_kinds, grid, items, R.bp_lds, P, R.L, st);
+    launch_bp_mode<16>(mode, R.bp_kinds, T.bp_grid, R.bp_total, R.bp_lds, P, R.L, st);
   CCPI_HIP(hipGetLastError());
 }
 
@@ -480,7 +476,7 @@ void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
            "," + std::to_string(G.nx) + "," + std::to_string(G.ny) + "," + std::to_string(G.nz) + ";";
   }
 
-  // autotune rows-per-lane and the FP / BP grids once per batch shape
+  // slices per BP item and the grids, tuned once per batch shape
   Tuned T{16, 0, 0};
   bool have = false;
   if (const char *env = std::getenv("CCPI_BATCH_TUNE")) {
@@ -502,48 +498,40 @@ void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
     }
   }
   if (!have) {
-    hipEvent_t e0, e1, e2;
-    CCPI_HIP(hipEventCreate(&e0));
-    CCPI_HIP(hipEventCreate(&e1));
-    CCPI_HIP(hipEventCreate(&e2));
-    float best = 1e30f;
-    for (int rc : {8, 16}) {
-      layout(R, rc, st);
-      // FP of d (scratch, contents irrelevant) and BP of r into s: the two
-      // projector launches of an iteration, outputs discarded; the first
-      // pair loads the kernels
-      Tuned cand{rc, 0, 0};
-      proj(R, cand, 0, st);
-      proj(R, cand, 1, st);
-      float fp_best = 1e30f, bp_best = 1e30f;
-      for (int mult : {0, 2, 4, 8}) {
-        const Tuned t{rc, mult * cu_count(), mult * cu_count()};
-        CCPI_HIP(hipEventRecord(e0, st));
-        proj(R, t, 0, st);
-        CCPI_HIP(hipEventRecord(e1, st));
-        proj(R, t, 1, st);
-        CCPI_HIP(hipEventRecord(e2, st));
-        CCPI_HIP(hipEventSynchronize(e2));
-        float fp_ms = 0.f, bp_ms = 0.f;
-        CCPI_HIP(hipEventElapsedTime(&fp_ms, e0, e1));
-        CCPI_HIP(hipEventElapsedTime(&bp_ms, e1, e2));
-        if (fp_ms < fp_best) {
-          fp_best = fp_ms;
-          cand.fp_grid = t.fp_grid;
-        }
-        if (bp_ms < bp_best) {
-          bp_best = bp_ms;
-          cand.bp_grid = t.bp_grid;
-        }
+    struct Events {
+      hipEvent_t a = nullptr, b = nullptr;
+      Events() {
+        CCPI_HIP(hipEventCreate(&a));
+        CCPI_HIP(hipEventCreate(&b));
       }
-      if (fp_best + bp_best < best) {
-        best = fp_best + bp_best;
-        T = cand;
+      ~Events() {
+        if (a) (void)hipEventDestroy(a);
+        if (b) (void)hipEventDestroy(b);
       }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    (void)hipEventDestroy(e2);
+    } ev;
+    auto time = [&](auto launch) {
+      CCPI_HIP(hipEventRecord(ev.a, st));
+      launch();
+      CCPI_HIP(hipEventRecord(ev.b, st));
+      CCPI_HIP(hipEventSynchronize(ev.b));
+      float ms = 0.f;
+      CCPI_HIP(hipEventElapsedTime(&ms, ev.a, ev.b));
+      return ms;
+    };
+    // FP of d (scratch, contents irrelevant) and BP of r into s, outputs
+    // discarded; the first launch of each loads its kernel
+    int rc = 16;
+    layout(R, rc, st);
+    if (R.fp_total > 0) proj_fp_items(R, 0, st);
+    T = tune_batch(
+        R.fp_total > 0, cu_count(),
+        [&](int slices) {
+          rc = slices;
+          layout(R, rc, st);
+          proj(R, Tuned{rc, 0, 0}, 1, st);
+        },
+        [&](int grid) { return time([&] { proj_fp_items(R, grid, st); }); },
+        [&](int grid) { return time([&] { proj(R, Tuned{rc, 0, grid}, 1, st); }); });
     std::lock_guard<std::mutex> lock(g_tune_mu);
     g_tuned[sig] = T;
   }

@@ -9,6 +9,7 @@
 #include <thread>
 #include <vector>
 
+#include "batch_tune.hpp"
 #include "grid.hpp"
 #include "kept.hpp"
 
@@ -139,12 +140,39 @@ static void refused_allocation() {
   EXPECT(Thing::live == 4);
 }
 
+// The BP's times alone choose the slices per item, whatever the FP's are; the
+// FP's grid is timed once each, and only where there are items to time.
+static void batch_tune() {
+  int rc = 0, fp_runs = 0;
+  // 16 slices are faster, at 4 workgroups per CU
+  auto bp = [&](int grid) { return (rc == 16 ? 7.0f : 8.0f) + (grid == 4 * 256 ? 0.f : 0.5f); };
+  auto items = [&](int r) { rc = r; };
+  for (bool have : {false, true})
+    for (float noise : {0.f, 100.f}) {
+      fp_runs = 0;
+      // an FP that was timed beside 16 slices would have spoilt them
+      auto fp = [&](int grid) {
+        fp_runs++;
+        return 9.0f + (rc == 16 ? noise : 0.f) + (grid == 2 * 256 ? 0.f : 1.f);
+      };
+      const ccpi::Tuned T = ccpi::tune_batch(have, 256, items, fp, bp);
+      EXPECT(T.rc == 16 && T.bp_grid == 4 * 256);
+      EXPECT(fp_runs == (have ? 4 : 0));
+      EXPECT(T.fp_grid == (have ? 2 * 256 : 0));
+    }
+  // no persistent grid where one workgroup per item is as fast
+  const ccpi::Tuned T =
+      ccpi::tune_batch(true, 256, items, [](int) { return 1.f; }, [](int) { return 1.f; });
+  EXPECT(T.rc == 8 && T.fp_grid == 0 && T.bp_grid == 0);
+}
+
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "grids")) grids();
   else if (!std::strcmp(what, "kept")) kept();
   else if (!std::strcmp(what, "kept_threads")) kept_threads();
   else if (!std::strcmp(what, "refused_allocation")) refused_allocation();
+  else if (!std::strcmp(what, "batch_tune")) batch_tune();
   else return 2;
   return failed;
 }
