@@ -124,6 +124,10 @@ struct ConeArgs {
 
 // ---- parallel beam plan layout ---------------------------------------------
 
+// Volumes of the parallel FP's shared walk: their byte offsets, and the one an
+// ended walk asks for, stay below 2^32.
+constexpr size_t kParShareBytes = 0xe0000000;
+
 struct ParArgs {
   int na, nh, nv, nx, ny, nz;
   int map_type;          // 1, 2, 4 (rows per slice) or 0 (general)

@@ -505,9 +505,6 @@ struct ParWalker {
   }
 };
 
-// Volumes of the shared walk: their byte offsets, and the one an ended walk
-// asks for, stay below 2^32.
-constexpr size_t kParShareBytes = 0xe0000000;
 inline bool par_share_fits(const ParArgs &g) {
   return g.map_type == 1 && sizeof(float) * (size_t)g.nx * g.ny * g.nz <= kParShareBytes;
 }

@@ -184,8 +184,9 @@ inline bool par_one_row_per_slice(const Geometry &g) {
 
 // Walk table of a parallel plan: built for FPs of fewer than
 // kParWalkTableWaves wavefronts (4 detector rows per lane; kParWalkTableWavesN
-// where rows and slices do not go one to one, whose lanes would each walk:
-// the table's 8 bytes per cell are read in their place) when its bound
+// where the shared walk does not take the FP - rows and slices not one to one,
+// or a volume past kParShareBytes - whose lanes would each walk: the table's 8
+// bytes per cell are read in their place) when its bound
 // (8 bytes per cell, at most nx + ny cells per ray, plus the ray offsets)
 // is within kParWalkTableBytes.
 constexpr size_t kParWalkTableBytes = size_t(4) << 30;
@@ -199,9 +200,10 @@ inline long long par_fp_waves(const Geometry &g) {
   return (long long)g.na * g.nh * ((g.nv + 4 * lr - 1) / (4 * lr)) * lr / 64;
 }
 inline bool par_walk_table_wanted(const Geometry &g) {
+  const bool shares =
+      par_one_row_per_slice(g) && g.n_vox() * sizeof(float) <= kParShareBytes;
   return par_walk_table_bound(g) <= kParWalkTableBytes &&
-         par_fp_waves(g) <
-             (par_one_row_per_slice(g) ? kParWalkTableWaves : kParWalkTableWavesN);
+         par_fp_waves(g) < (shares ? kParWalkTableWaves : kParWalkTableWavesN);
 }
 
 std::shared_ptr<ConePlan> cone_plan(const Geometry &g, hipStream_t st);
