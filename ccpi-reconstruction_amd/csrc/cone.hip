@@ -403,8 +403,10 @@ __device__ inline Acc fp_inside(const FpRow &R, FpPos &P, const float *vol, int 
   return acc;
 }
 
-// Segments of one ray for the wave's rows, up to me, kFpGroup at a time: all
-// their gathers are issued before the in-order accumulation (the sum order
+// Segments of one ray for the wave's rows, up to me: of each, the row's two
+// slices (c2D.cpp:104-143, 153-187) weighted by their alpha lengths; slices
+// outside [0, nz) read 0 through the buffer range check.  kFpGroup segments at
+// a time: all their gathers are issued before the in-order accumulation (the sum order
 // is the reference's), and the next group's entries are loaded while they
 // are in flight.  The last group may read entries past `me` (the tables are
 // padded); what lies past it is not added.  The wave stops once the segment
@@ -420,9 +422,7 @@ __device__ inline Acc fp_inside(const FpRow &R, FpPos &P, const float *vol, int 
 // column's byte offset comes from the table (20 scalar instructions per
 // segment before, 6 now).  512^3 (720 x 768^2) 80.7 -> 60.0 ms, 256^3 (360 x
 // 384^2) 4.99 -> 4.07, XTek wide cone 384^3 16.1 -> 7.6, bit-identical.
-// One xy segment [a0, a1] of a column, ai = a0 / voxel z size: the row's two
-// slices (c2D.cpp:104-143, 153-187) weighted by their alpha lengths.  Slices
-// outside [0, nz) read 0 through the buffer range check.
+//
 // DIR: -1 / +1 every row of the wave under / over the source (the second
 // slice is one below / above the first and the boundary plane k / k + 1),
 // 0 both kinds.  EDGE: floor-form rows among them.

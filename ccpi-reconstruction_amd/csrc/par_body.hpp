@@ -670,17 +670,6 @@ __device__ inline double par_fp_shared(const ParArgs &g, int a, int h0, int v0, 
   return ss;
 }
 
-// One thread of the FP, one ray per lane: ray bx * 256 + tid, rows
-// [by * RC, by * RC + RC).
-template <int RC>
-__device__ inline double par_fp_thread(const ParArgs &g, int bx, int by, int tid,
-                                       const float *__restrict__ vol,
-                                       float *__restrict__ sino, bool acc_in) {
-  const int r = bx * 256 + tid;
-  if (r >= g.na * g.nh) return 0.0;
-  return par_fp_rows<RC>(g, r, by * RC, vol, sino, acc_in);
-}
-
 // FP, ray-shared layout: `lr` lanes (a power of two, at most 16) share one
 // ray, each taking 4 consecutive detector rows, so the lanes of a ray read
 // one contiguous run of every crossed column.  Block bx holds rays
