@@ -431,11 +431,11 @@ int cu_count() {
 
 void run_pb_cgls_batched(const std::vector<Geometry> &geoms, float *const *b,
                          float *const *x, int iters, double *norms_out, hipStream_t caller) {
+  if (geoms.empty()) return;
   WorkspaceLease lease;
   std::vector<char> tables;
   BatchRun R{*lease};
   R.count = (int)geoms.size();
-  if (R.count == 0) return;
   CCPI_HIP(hipStreamSynchronize(caller));
   hipStream_t st;
   CCPI_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
