@@ -100,6 +100,7 @@ def run(workload: str, iters: int = 5, calibrate: bool = False):
       wide      the same scan through the XTek volume rule (768^3 of
                 0.811 mm, the phased BP);
       cfg1      parallel 256 x 256 x 16, 180 angles, 367 x 16 detector;
+      par512    parallel 512 x 512 x 32, 360 angles, 725 x 32 detector;
       batch64   the 64 uneven parallel problems, plain (one at a time);
       batch64b  the same problems, batched (one persistent launch per step).
     ``calibrate`` first copies 1 GiB device to device (the known-size kernel
@@ -114,14 +115,16 @@ def run(workload: str, iters: int = 5, calibrate: bool = False):
         torch.empty_like(src).copy_(src)
         torch.cuda.synchronize()
         del src
-    if workload in ("cone512", "wide", "cfg1"):
+    if workload in ("cone512", "wide", "cfg1", "par512"):
         if workload == "cone512":
             g = W.cone_geometry(**W.CONE_512)
         elif workload == "wide":
             ang = np.linspace(0, 360, 720, endpoint=False).astype(np.float32)
             g = ins.xtek_setup((720, 768, 768), ang, 1, -500.0, 500.0, 1.0, 1.0, 128.0).geometry
-        else:
+        elif workload == "cfg1":
             g = W.parallel_geometry(256, 16, 180, 367)
+        else:
+            g = W.parallel_geometry(512, 32, 360, 725)
         gen = torch.Generator(device="cuda").manual_seed(7)
         b = torch.rand(g.sino_shape, device="cuda", generator=gen)
         cgls(g, b, iters)
