@@ -406,16 +406,16 @@ __device__ inline Acc fp_inside(const FpRow &R, FpPos &P, const float *vol, int 
 // Segments of one ray for the wave's rows, up to me: of each, the row's two
 // slices (c2D.cpp:104-143, 153-187) weighted by their alpha lengths; slices
 // outside [0, nz) read 0 through the buffer range check.  kFpGroup segments at
-// a time: all their gathers are issued before the in-order accumulation (the sum order
-// is the reference's), and the next group's entries are loaded while they
-// are in flight.  The last group may read entries past `me` (the tables are
+// a time: all their gathers are issued before the in-order accumulation (the
+// sum order is the reference's), and the next group's entries are loaded while
+// they are in flight.  The last group may read entries past `me` (the tables are
 // padded); what lies past it is not added.  The wave stops once the segment
 // start passes every row's exit parameter (amax_bits: a non-negative
 // float's bits, so the integer compare is the float compare).
 //
-// Bound: VALU issue (12 instructions per segment and wave inside the volume,
-// 15 to 17 elsewhere; 87 % busy at 512^3) and the L1's accesses together
-// (TA 99 % busy).  The two slices of a segment are two dword loads: 64 rows
+// Bound: the texture path (at 512^3 TA 98 and TD 100 % busy), with up to 87 %
+// of the cycles of VALU issue (12 instructions per segment and wave inside the
+// volume, 15 to 17 elsewhere).  The two slices of a segment are two dword loads: 64 rows
 // of one dword are near-contiguous and take about 9 L1 accesses, both in one
 // 8-byte load 15 (512^3 67.3 ms against 61.2).  One pair of wide scalar loads
 // per group replaces 16 narrow ones that each waited for the last, and the
@@ -884,9 +884,9 @@ __device__ inline BpSlot bp_slot(const ConeArgs &g, int v, int pass, bool one_se
 }
 
 // S (at most 4) consecutive rows of one lane in one load.  One 4-byte load
-// per row, 4 S bytes apart between lanes, asked L1 for S times the lines: it
-// was busy 94 % of the time at S = 2 (512^3 cone 88.4 -> 83.5 ms, 256^3 6.15
-// -> 5.88, 64 x 64 x 48 0.066 -> 0.063).
+// per row, 4 S bytes apart between lanes, asked L1 for S times the lines
+// (512^3 cone, S = 2, 88.4 -> 83.5 ms, 256^3 6.15 -> 5.88, 64 x 64 x 48 0.066
+// -> 0.063; the texture data path is still 96 % busy at 512^3).
 template <int S>
 __device__ inline void bp_load_rows(__amdgpu_buffer_rsrc_t row, int at, int base, float *p) {
   if constexpr (S == 1) {

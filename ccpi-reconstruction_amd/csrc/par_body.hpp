@@ -409,8 +409,8 @@ __device__ inline double par_fp_rows(const ParArgs &g, int r, int v0,
 // rows per ray and NS rays per lane.  Cells are par_walk_groups' (the same
 // steps and lengths), added in the walk's order.
 //
-// Bound: the gathers' 64 bytes per cycle and CU from L1 (TD 79 % busy, VALU
-// 62 % at 512 x 512 x 32, 360 angles).  With every lane walking, 8 lanes
+// Bound: the gathers' 64 bytes per cycle and CU from L1 (512 x 512 x 32, 360
+// angles: TD 84 % busy, TA 78, VALU issue up to 65 % of the cycles).  With every lane walking, 8 lanes
 // repeated each ray's double arithmetic (35 instructions per cell against 10
 // to gather and sum it): 512 x 512 x 32 1.51 -> 0.67 ms, 383 x 383 x 29 (180
 // angles) 0.52 -> 0.23, 256 x 256 x 16 (180) 0.135 -> 0.080.  A wavefront that
@@ -912,9 +912,9 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // one coalesced copy per tile instead of each lane re-reading its columns'
 // rows, and with the columns' positions; every lane then weighs its own
 // column's footprint (the reference's FP64 arithmetic) on the staged rows.
-// Bound by vector issue (busy all the time at 512 x 512 x 32), about 115
-// instructions per column and angle of which 64 are the 16 slices' products
-// and sums.  So there are two blocks of LDS and the next one's reads go
+// Bound by vector issue (at 512 x 512 x 32 up to 86 % of the cycles, LDS 61 %,
+// half of it bank conflicts), 123 instructions per wavefront and angle of which
+// 64 are the 16 slices' products and sums.  So there are two blocks of LDS and the next one's reads go
 // straight there while this one is summed (one barrier a block, no register
 // in between), spans are found 256 angles at a time, tables are scalar loads,
 // and where a voxel's shadow is under two columns wide (pixels about as wide
