@@ -483,15 +483,6 @@ __device__ inline Acc fp_run(const FpRow &R, FpPos P, const float *vol, int nz, 
   return acc;
 }
 
-// Ray tiles of the FP: consecutive workgroups of one XCD take a tile of
-// adjacent angles x adjacent rays, whose walks cross mostly the same columns
-// at the same time, so the columns are read from that XCD's L2.  512^3, ms
-// per FP and bytes fetched from beyond L2: rays dealt to the XCDs in turn
-// 83 / 601 GB; tiles of 16 x 16 67.7, 1 x 64 78.4, 8 x 32 72.7, 32 x 8 66.1;
-// with the loads as they are now 32 x 8 60.8, 64 x 8 60.0 / 203 GB, 128 x 8
-// 59.7, 128 x 4 60.6; 256^3 4.07 to 4.10 for all four.
-constexpr int kFpTileA = 64, kFpTileH = 8;
-
 // One workgroup per ray and block of detector rows, one row per lane.  Acc
 // as fp_run; with double the result is rounded once, after the d_conv
 // scaling.
@@ -503,15 +494,12 @@ __global__ __launch_bounds__(kFpRows) void cone_fp_kernel(
   extern __shared__ float smem[];
   const int nrays = g.na * g.nh;
   // workgroup -> (row block, angle, column) through the XCD's tile
-  const int wgs = g.fp_tile_a * kFpTileH;
-  const int id = wg_index(), xcd = id % kXcds, local = id / kXcds;
-  const int tile = (local / wgs) * kXcds + xcd, within = local % wgs;
-  const int nth = (g.nh + kFpTileH - 1) / kFpTileH;
-  const int nta = (g.na + g.fp_tile_a - 1) / g.fp_tile_a;
-  const int rb = tile / (nth * nta), tah = tile - rb * (nth * nta);
-  const int a = (tah / nth) * g.fp_tile_a + within / kFpTileH;
-  const int h = (tah % nth) * kFpTileH + within % kFpTileH;
-  if (rb >= g.fp_blocks || a >= g.na || h >= g.nh) return;
+  const int tile = (int)(blockIdx.y * kXcds + blockIdx.x % kXcds);
+  const int within = (int)(blockIdx.x / kXcds), rb = (int)blockIdx.z;
+  const int nth = (g.nh + kFpTileH - 1) / kFpTileH, ta = tile / nth;
+  const int a = ta * g.fp_tile_a + within / kFpTileH;
+  const int h = (tile - ta * nth) * kFpTileH + within % kFpTileH;
+  if (a >= g.na || h >= g.nh) return;
   const int r = a * g.nh + h;
   // slice planes, clamped at both ends: plane q at s_vz[q + kFpPad]
   for (int q = threadIdx.x; q < g.nz + 1 + 2 * kFpPad; q += blockDim.x)
@@ -1548,9 +1536,7 @@ void cone_build_plan(ConePlan &P, hipStream_t st) {
     const int waves = (nv + 63) / 64, per = kFpRows / 64;
     A.fp_blocks = (waves + per - 1) / per;
     A.fp_threads = 64 * ((waves + A.fp_blocks - 1) / A.fp_blocks);
-    // angles per ray tile: at most kFpTileA, spread evenly over the tiles
-    const int nta = (na + kFpTileA - 1) / kFpTileA;
-    A.fp_tile_a = (na + nta - 1) / nta;
+    A.fp_tile_a = cone_fp_tiles(na, nh).angles;
     A.fp_big = G.n_vox() * sizeof(float) > 0xffffffffull ? 1 : 0;
   }
 
@@ -1742,11 +1728,13 @@ template <bool BIG, class Acc>
 static void cone_fp_launch(const ConePlan &P, const float *vol, float *sino, hipStream_t st,
                            bool acc_in, double *norm) {
   const ConeArgs &A = P.args;
-  // ray tiles of every row block, dealt to the XCDs in turn
-  const long long tiles = (long long)A.fp_blocks * ((A.na + A.fp_tile_a - 1) / A.fp_tile_a) *
-                          ((A.nh + kFpTileH - 1) / kFpTileH);
-  const long long blocks = (tiles + kXcds - 1) / kXcds * kXcds * (A.fp_tile_a * kFpTileH);
-  const dim3 grid = wg_dim3(blocks, A.fp_threads, "cone FP: too many rays");
+  // x: a workgroup of each XCD's tile in turn, so a workgroup's number modulo 8,
+  // its XCD, is x modulo 8; y: the next eight tiles; z: row blocks
+  const long long tiles = cone_fp_tiles(A.na, A.nh).tiles;
+  CCPI_REQUIRE(tiles < (1LL << 31) - kXcds, CCPI_E_LIMIT, "cone FP: too many rays");
+  const long long eights = (tiles + kXcds - 1) / kXcds;
+  const dim3 grid((unsigned)(kXcds * A.fp_tile_a * kFpTileH), (unsigned)eights,
+                  (unsigned)A.fp_blocks);
   const size_t lds = sizeof(float) * (size_t)(A.nz + 1 + 2 * kFpPad);
   hipLaunchKernelGGL((cone_fp_kernel<BIG, Acc>), grid, dim3(A.fp_threads), lds, st, A,
                      P.rays.as<ConeRay>(), P.ents.as<ConeEnt>(), P.eai.as<float>(), vol, sino,

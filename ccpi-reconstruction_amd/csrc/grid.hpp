@@ -2,6 +2,8 @@
 // types: the launchers and the CPU checks share it).
 #pragma once
 
+#include <algorithm>
+
 namespace ccpi {
 
 constexpr int kXcds = 8;
@@ -23,6 +25,31 @@ inline WgGrid wg_grid(long long blocks, int threads) {
   if (blocks >= (1LL << 31) - row) return {0, 0};
   if (blocks * threads < (1LL << 32)) return {(unsigned)blocks, 1};
   return {(unsigned)row, (unsigned)((blocks + row - 1) / row)};
+}
+
+// Ray tiles of the cone FP: consecutive workgroups of one XCD take a tile of
+// adjacent angles x adjacent rays, whose walks cross mostly the same columns
+// at the same time, so the columns are read from that XCD's L2.  512^3, ms
+// per FP and bytes fetched from beyond L2: rays dealt to the XCDs in turn
+// 83 / 601 GB; tiles of 16 x 16 67.7, 1 x 64 78.4, 8 x 32 72.7, 32 x 8 66.1;
+// with the loads as they are now 32 x 8 60.8, 64 x 8 60.0 / 203 GB, 128 x 8
+// 59.7, 128 x 4 60.6; 256^3 4.07 to 4.10 for all four.
+// A tile has at most kFpTileA angles, and fewer where that leaves an XCD less
+// than kFpTiles tiles: with 64 angles, 58 angles x 13 columns were one tile
+// each for four XCDs and none for the others (64 x 130 x 12, 447 rows 0.0189
+// ms before the tiles, 0.0253 with 64 angles, 0.0156 now), 103 x 19 columns 3
+// for some and 2 for others (57 x 62 x 29, 515 rows 0.025, 0.028, 0.020).
+constexpr int kFpTileA = 64, kFpTileH = 8, kFpTiles = 16;
+struct RayTiles {
+  int angles;        // per tile
+  long long tiles;
+};
+inline RayTiles cone_fp_tiles(int na, int nh) {
+  const int nth = (nh - 1) / kFpTileH + 1;
+  const int nta = std::max((na - 1) / kFpTileA + 1,
+                           std::min(na, (kXcds * kFpTiles - 1) / nth + 1));
+  const int angles = (na - 1) / nta + 1;
+  return {angles, (long long)((na - 1) / angles + 1) * nth};
 }
 
 }  // namespace ccpi

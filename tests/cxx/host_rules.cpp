@@ -41,6 +41,27 @@ static void grids() {
   }
 }
 
+// Live rays of the cone FP per XCD: where there are enough rays to share, no
+// XCD has much more than its share of the rays with the last column tile full.
+static void cone_tiles() {
+  for (int na : {1, 5, 33, 58, 64, 65, 90, 103, 146, 194, 360, 720})
+    for (int nh : {2, 9, 13, 17, 19, 64, 96, 283, 384, 768}) {
+      const ccpi::RayTiles T = ccpi::cone_fp_tiles(na, nh);
+      const int nth = (nh + ccpi::kFpTileH - 1) / ccpi::kFpTileH;
+      EXPECT(T.angles >= 1 && T.angles <= ccpi::kFpTileA && T.tiles % nth == 0);
+      EXPECT(T.tiles / nth * T.angles >= na && (T.tiles / nth - 1) * T.angles < na);
+      long long per[ccpi::kXcds] = {}, most = 0;
+      for (long long t = 0; t < T.tiles; t++) {
+        const long long a0 = t / nth * T.angles, h0 = t % nth * ccpi::kFpTileH;
+        per[t % ccpi::kXcds] += std::min<long long>(T.angles, na - a0) *
+                                std::min<long long>(ccpi::kFpTileH, nh - h0);
+      }
+      for (long long p : per) most = std::max(most, p);
+      if ((long long)na * nth >= ccpi::kXcds * ccpi::kFpTiles)
+        EXPECT(most * ccpi::kXcds <= 1.15 * na * nth * ccpi::kFpTileH);
+    }
+}
+
 struct Thing {
   static std::atomic<int> live;
   int id;
@@ -169,6 +190,7 @@ static void batch_tune() {
 int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "grids")) grids();
+  else if (!std::strcmp(what, "cone_tiles")) cone_tiles();
   else if (!std::strcmp(what, "kept")) kept();
   else if (!std::strcmp(what, "kept_threads")) kept_threads();
   else if (!std::strcmp(what, "refused_allocation")) refused_allocation();

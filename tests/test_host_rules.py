@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["grids", "kept", "kept_threads", "refused_allocation",
+@pytest.mark.parametrize("check", ["grids", "kept", "kept_threads", "refused_allocation", "cone_tiles",
                                    "batch_tune"])
 def test_host_rule(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True)
