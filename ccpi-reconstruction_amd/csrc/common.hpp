@@ -107,7 +107,8 @@ struct ConeArgs {
   float zb, zt;          // volume bottom / top relative to source z
   const float *alim;     // [nv] walk parameter where row v leaves the volume's
                          // z range (>= 2 where it never does)
-  const float *ain;      // [nv] walk parameter until which row v is a slice inside
+  const float *wlim;     // [2 ceil(nv / 64)] per 64 rows: walk parameter until which all are a slice
+                         // inside, and the largest alim
   float pzbz, pzbz1, inv_dz;
   float pzdv, z1, znm;   // BP safe-row bounds (c2D.cpp:993-1000)
   double vx, vy, dx, dy; // volume xy origin and voxel size

@@ -116,13 +116,13 @@ struct SharedScratch {
 struct ConePlan {
   Geometry g;
   ConeArgs args{};
-  DeviceBuffer atab, hpix, hrange, dz, iz, vz, dconv, offs, rays, ents, eai, alim, ain;
+  DeviceBuffer atab, hpix, hrange, dz, iz, vz, dconv, offs, rays, ents, eai, alim, wlim;
   DeviceBuffer bpcol, bprec;  // backprojection lists
   SharedScratch scratch;      // BP scratch of callers without a workspace
   uint64_t n_entries = 0;
   size_t bytes() const {
     return atab.bytes + hpix.bytes + hrange.bytes + dz.bytes + iz.bytes +
-           vz.bytes + dconv.bytes + offs.bytes + rays.bytes + ents.bytes + eai.bytes + alim.bytes + ain.bytes +
+           vz.bytes + dconv.bytes + offs.bytes + rays.bytes + ents.bytes + eai.bytes + alim.bytes + wlim.bytes +
            bpcol.bytes + bprec.bytes + scratch.bytes();
   }
 };
