@@ -1,8 +1,9 @@
-// How a launch's workgroups are laid over a grid (host arithmetic, no HIP
-// types: the launchers and the CPU checks share it).
+// How a launch's workgroups are laid over a grid and over a CU's LDS (host
+// arithmetic, no HIP types: the launchers and the CPU checks share it).
 #pragma once
 
 #include <algorithm>
+#include <cstddef>
 
 namespace ccpi {
 
@@ -50,6 +51,31 @@ inline RayTiles cone_fp_tiles(int na, int nh) {
                            std::min(na, (kXcds * kFpTiles - 1) / nth + 1));
   const int angles = (na - 1) / nta + 1;
   return {angles, (long long)((na - 1) / angles + 1) * nth};
+}
+
+// LDS of the parallel tiled BP per angle of a block, two blocks: hmax columns
+// of `slices` rows, their positions and the span.
+inline std::size_t par_bp_angle_bytes(int hmax, int slices) {
+  return 2 * ((std::size_t)hmax * (sizeof(float) * slices + sizeof(double)) + 2 * sizeof(int));
+}
+// LDS of one workgroup: the blocks and the spans of 256 angles.
+inline std::size_t par_bp_tile_bytes(int hmax, int slices, int ab) {
+  return par_bp_angle_bytes(hmax, slices) * (std::size_t)ab + 256 * 2 * sizeof(int);
+}
+// Angles per block: at most 4 (a wavefront stages one each), and as many as
+// leave the CU's 160 KB, handed out in units of 1280 bytes, for the five
+// workgroups that the registers allow (128 bytes are the norm's); or else one.
+// With 32 KB of blocks only four fitted where pixels are half a voxel or a
+// quarter with 8 slices: 237 x 237 x 13, 133 angles, pixels of half a voxel
+// 0.106 ms before there were two blocks, 0.121 with four angles (30016 bytes),
+// 0.099 with three; 458 x 224 x 2, 317 angles, a quarter 0.44, 0.53, 0.42.
+// Fewer than fit lose: 566 x 566 x 16, 73 angles, a quarter 0.52 with two (27968
+// bytes), 0.56 with one.
+constexpr std::size_t kParBpLds = 25 * 1280;
+inline int par_bp_block_angles(int hmax, int slices) {
+  int n = 4;
+  while (n > 1 && par_bp_tile_bytes(hmax, slices, n) + 128 > kParBpLds) n--;
+  return n;
 }
 
 }  // namespace ccpi

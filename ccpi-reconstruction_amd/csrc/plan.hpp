@@ -139,21 +139,6 @@ struct ParBpShape {
   int groups = 1;    // angle groups summed through scratch partials
 };
 
-// LDS of the tiled BP per angle of a block, two blocks: hmax columns of
-// `slices` rows, their positions and the span; and the angles per block, at
-// most 4 (a wavefront stages one each), that fit 32 KB or else one.
-inline size_t par_bp_angle_bytes(int hmax, int slices) {
-  return 2 * ((size_t)hmax * (sizeof(float) * slices + sizeof(double)) + 2 * sizeof(int));
-}
-inline int par_bp_block_angles(int hmax, int slices) {
-  const size_t n = (32 * 1024) / par_bp_angle_bytes(hmax, slices);
-  return n < 1 ? 1 : n > 4 ? 4 : (int)n;
-}
-// LDS of one workgroup: the blocks and the spans of 256 angles.
-inline size_t par_bp_tile_bytes(int hmax, int slices, int ab) {
-  return par_bp_angle_bytes(hmax, slices) * (size_t)ab + 256 * 2 * sizeof(int);
-}
-
 struct ParPlan {
   Geometry g;
   ParArgs args{};

@@ -62,6 +62,23 @@ static void cone_tiles() {
     }
 }
 
+// The tiled parallel BP's blocks leave room for five workgroups on a CU (160 KB,
+// handed out 1280 bytes at a time, with 128 bytes of the kernel's own) wherever
+// more than one angle is staged, and no angle less than fits is staged.
+static void bp_blocks() {
+  for (int slices : {8, 16})
+    for (int hmax = 7; hmax <= 1023; hmax++) {
+      const int ab = ccpi::par_bp_block_angles(hmax, slices);
+      auto five = [&](int n) {
+        return 5 * ((ccpi::par_bp_tile_bytes(hmax, slices, n) + 128 + 1279) / 1280 * 1280) <=
+               160 * 1024;
+      };
+      EXPECT(ab >= 1 && ab <= 4);
+      EXPECT(ab == 1 || five(ab));
+      EXPECT(ab == 4 || !five(ab + 1));
+    }
+}
+
 struct Thing {
   static std::atomic<int> live;
   int id;
@@ -191,6 +208,7 @@ int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "grids")) grids();
   else if (!std::strcmp(what, "cone_tiles")) cone_tiles();
+  else if (!std::strcmp(what, "bp_blocks")) bp_blocks();
   else if (!std::strcmp(what, "kept")) kept();
   else if (!std::strcmp(what, "kept_threads")) kept_threads();
   else if (!std::strcmp(what, "refused_allocation")) refused_allocation();

@@ -18,8 +18,8 @@ def program(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("check", ["grids", "kept", "kept_threads", "refused_allocation", "cone_tiles",
-                                   "batch_tune"])
+@pytest.mark.parametrize("check", ["grids", "kept", "kept_threads", "refused_allocation",
+                                   "cone_tiles", "bp_blocks", "batch_tune"])
 def test_host_rule(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
