@@ -448,7 +448,7 @@ static ParFpForm par_fp_form(const ParArgs &A) {
 // the launch within kParTableWaves wavefronts (384 x 384 x 2, 180 angles:
 // 0.204 / 0.107 / 0.108 ms with 4 / 8 / 8 lanes at limits of 8192 / 16384 /
 // 32768; 200 x 200 x 16, 120 angles: 0.059 / 0.057 / 0.060 with 2 / 4 / 8).
-// Volumes that the shared walk does not take (the only ones here from
+// Volumes past the shared walk's size and short rays (all that is here from
 // kParWalkTableWaves on) have one lane from there on: 1025 x 1025 x 900, 380
 // columns, 2 angles (2850 waves) 0.63 with 1, 0.70 with 4, 0.67 without a
 // table; 1 angle (1425) 0.44 with 1, 0.39 with 8.

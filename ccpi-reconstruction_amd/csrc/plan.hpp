@@ -171,7 +171,8 @@ inline bool par_one_row_per_slice(const Geometry &g) {
 // kParWalkTableWaves wavefronts (4 detector rows per lane; kParWalkTableWavesN
 // where the shared walk does not take the FP - rows and slices not one to one,
 // or a volume past kParShareBytes - whose lanes would each walk: the table's 8
-// bytes per cell are read in their place) when its bound
+// bytes per cell are read in their place; and where it would walk short rays for
+// 16 lanes each, mostly start and barriers) when its bound
 // (8 bytes per cell, at most nx + ny cells per ray, plus the ray offsets)
 // is within kParWalkTableBytes.
 constexpr size_t kParWalkTableBytes = size_t(4) << 30;
@@ -184,9 +185,19 @@ inline long long par_fp_waves(const Geometry &g) {
   const int lr = par_fp_lanes_per_ray(g.nv);
   return (long long)g.na * g.nh * ((g.nv + 4 * lr - 1) / (4 * lr)) * lr / 64;
 }
+// Short rays: volumes whose nx and ny have a harmonic mean of at most
+// kParShortRay cells.  More than 32 rows, ms table / shared: 20 x 20 x 122, 387
+// angles x 28 columns 0.017 / 0.030; 30 x 30 x 35, 301 x 75 0.016 / 0.026; 31 x 31
+// x 116, 113 x 44 0.014 / 0.016; past the line either wins: 25 x 82 x 98 (38
+// cells), 13 x 410 0.022 / 0.031; 27 x 66 x 51 (38), 228 x 93 0.032 / 0.027; 32 x
+// 60 x 43 (42), 310 x 60 0.030 / 0.021.  Up to 32 rows, 8 lanes a ray: 37 x 37 x
+// 18, 386 x 92 0.024 / 0.021.
+constexpr int kParShortRay = 32;
 inline bool par_walk_table_wanted(const Geometry &g) {
-  const bool shares =
-      par_one_row_per_slice(g) && g.n_vox() * sizeof(float) <= kParShareBytes;
+  const bool short_rays = par_fp_lanes_per_ray(g.nv) == 16 &&
+                          2.0 * g.nx * g.ny <= (double)kParShortRay * (g.nx + g.ny);
+  const bool shares = par_one_row_per_slice(g) &&
+                      g.n_vox() * sizeof(float) <= kParShareBytes && !short_rays;
   return par_walk_table_bound(g) <= kParWalkTableBytes &&
          par_fp_waves(g) < (shares ? kParWalkTableWaves : kParWalkTableWavesN);
 }
