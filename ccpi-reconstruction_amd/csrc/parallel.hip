@@ -452,13 +452,20 @@ static ParFpForm par_fp_form(const ParArgs &A) {
 // kParWalkTableWaves on) have one lane from there on: 1025 x 1025 x 900, 380
 // columns, 2 angles (2850 waves) 0.63 with 1, 0.70 with 4, 0.67 without a
 // table; 1 angle (1425) 0.44 with 1, 0.39 with 8.
+// Rays that cross few cells (nx + ny up to kParFewCells) have a quarter of that:
+// eight cells each for eight lanes are most of them: 20 x 20 x 32, 255 angles x 50
+// columns 0.0083 ms with one lane walking the table, 0.0109 with eight, 0.0086
+// with two; 21 x 21 x 127, 89 x 29 0.0118, 0.0128 and 0.0092; 51 x 51 x 85 (102), 56
+// x 63 0.022, 0.0147 and 0.0154.
 constexpr long long kParTableWaves = 16384;
+constexpr int kParFewCells = 64;
 static int par_fp_cell_lanes(const ParArgs &A, int lr) {
   const long long rows = (A.nv + 4 * lr - 1) / (4 * lr);
   const long long lanes = (long long)A.na * A.nh * rows * lr;
   if (lanes / 64 >= kParWalkTableWaves) return 1;
   int cl = 8;
-  while (cl > 1 && lanes * cl / 64 > kParTableWaves) cl /= 2;
+  const long long most = A.nx + A.ny <= kParFewCells ? kParTableWaves / 4 : kParTableWaves;
+  while (cl > 1 && lanes * cl / 64 > most) cl /= 2;
   return cl;
 }
 

@@ -1,6 +1,7 @@
 """Which parallel plans of one row per slice hold a walk table (GPU test).
 
-Below 2400 wavefronts all do; up to 8192 those of short rays (a harmonic mean of
+Below 2400 wavefronts all do, with up to 8 lanes on a ray's cells (volumes of nx
++ ny up to 64 cells fewer: 1, 2 and 4 here); up to 8192 those of short rays (a harmonic mean of
 nx and ny up to 32 cells) with more than 32 rows.  The plan's bytes show the
 table (8 bytes per cell of every ray); the projection is the oracle's within
 1e-5 of the maximum, as for the other FP forms, from zero and onto an output.
@@ -26,6 +27,9 @@ def _pb(nx, ny, nz, na, nh):
 # geometry, wavefronts at least and below, whether a table is held
 CASES = {
     "few_waves": (_pb(64, 64, 40, 60, 91), (1, 2400), True),
+    "few_cells_one_lane": (_pb(20, 21, 40, 290, 31), (2050, 2400), True),
+    "few_cells_two_lanes": (_pb(20, 20, 32, 250, 50), (1025, 2049), True),
+    "few_cells_four_lanes": (_pb(25, 25, 36, 142, 25), (513, 1025), True),
     "short_33_rows": (_pb(32, 32, 33, 170, 70), (2400, 8192), True),
     "short_130_rows": (_pb(29, 35, 130, 90, 60), (2400, 8192), True),
     "short_long_side": (_pb(16, 700, 40, 90, 120), (2400, 8192), True),
