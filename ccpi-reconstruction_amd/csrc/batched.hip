@@ -183,7 +183,7 @@ __attribute__((amdgpu_waves_per_eu(batch_min_waves<MODE, BPK>(), 8))) void batch
     double ss;
     if (BPK == 1 || (BPK == 3 && B.bp_tiled)) {
       ss = par_bp_tile<RC, float, true>(g, local % B.bp_nbx, local / B.bp_nbx, 0, g.na,
-                                        B.bp_hmax, B.bp_ab, false, r, dst, smem,
+                                        B.bp_hmax, B.bp_ab, false, r, dst, smem, true,
                                         B.bp_groups);
     } else {
       ss = par_bp_thread<RC>(g, local % B.bp_nbx, local / B.bp_nbx, threadIdx.x, r, dst,

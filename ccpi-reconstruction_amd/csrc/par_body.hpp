@@ -912,7 +912,7 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // one coalesced copy per tile instead of each lane re-reading its columns'
 // rows, and with the columns' positions; every lane then weighs its own
 // column's footprint (the reference's FP64 arithmetic) on the staged rows.
-// Bound by vector issue (at 512 x 512 x 32 up to 86 % of the cycles, LDS 61 %,
+// Bound by vector issue (at 512 x 512 x 32 up to 87 % of the cycles, LDS 61 %,
 // half of it bank conflicts), 123 instructions per wavefront and angle of which
 // 64 are the 16 slices' products and sums.  So there are two blocks of LDS and the next one's reads go
 // straight there while this one is summed (one barrier a block, no register
@@ -921,10 +921,16 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // as a voxel or wider) two columns are weighed without a loop, a last column
 // or tests that even columns answer.  With the rows staged through registers
 // between two barriers and a loop over positions in global memory it took:
-// 512 x 512 x 32, 360 angles 1.40 ms, now 0.68; 383 x 383 x 29, 180 angles
-// 0.44, now 0.24; 256 x 256 x 16, 180 angles 0.116, now 0.066; 64 x 64 x 1, 90
+// 512 x 512 x 32, 360 angles 1.40 ms, now 0.66; 383 x 383 x 29, 180 angles
+// 0.43, now 0.23; 256 x 256 x 16, 180 angles 0.116, now 0.061; 64 x 64 x 1, 90
 // angles 0.027, now 0.019; with the staging alone 0.89, 0.31, 0.081 and
-// 0.021.  Angles are visited in order, so with
+// 0.021.  Of few angles the sums are the least part: there the set-up, whose
+// code each launch fetches anew, and the writes count, so an accumulating
+// call's reads are behind one test, and four slices that all have a row are
+// written at once.  Slice by slice, each under its own tests, 55 x 358 x 59, 11
+// angles took 0.060 ms (0.043 before there was a two-column form), now 0.025;
+// 200 x 200 x 64, 20 angles 0.075, now 0.035; 256 x 256 x 16, 180 angles 0.067,
+// now 0.061.  Angles are visited in order, so with
 // one angle group the result is bit-identical to par_bp_kernel; with G
 // groups (blockIdx.z) each group writes its partial sums of its angle range
 // to part[group] and par_bp_sum_kernel adds them in group order.
@@ -933,8 +939,8 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // (it synchronises the workgroup): tile `tile` (16 x 16 columns, row-major
 // over the column grid), slices [zc * R, zc * R + R), angles [a_begin,
 // a_end).  The result goes to `dst` (a volume-layout array), added to its
-// contents when acc_in.  Returns the thread's sum of squares of the values
-// it wrote (0 for threads outside the volume).  smem: par_bp_tile_bytes,
+// contents when acc_in.  norm: returns the thread's sum of squares of the
+// values it wrote (0 for threads outside the volume).  smem: par_bp_tile_bytes,
 // 16-byte aligned; a caller with another item to do synchronises first.
 // FOLD (the batched kernel's tiled items; acc_in must be false): the
 // angles are split into `groups` ranges as par_bp_lds_kernel splits them,
@@ -947,7 +953,8 @@ constexpr int kParBpNarrow = 1 << 30;
 template <int R, class Acc, bool FOLD = false>
 __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, int a_end,
                               int hmax, int ab, bool acc_in, const float *__restrict__ sino,
-                              float *__restrict__ dst_vol, float *smem, int groups = 1) {
+                              float *__restrict__ dst_vol, float *smem, bool norm,
+                              int groups = 1) {
   static_assert(R % 4 == 0, "rows are read 4 at a time");
   constexpr int Q4 = R / 4;
   // two buffers of a block's rows, column positions and spans
@@ -968,8 +975,12 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
   Acc acc[R];
   CCPI_GLOBAL float *__restrict__ vcol = gmem(dst_vol) + colid * nz + k0;
 #pragma unroll
-  for (int q = 0; q < R; q++)
-    acc[q] = (!FOLD && acc_in && active && q < nk) ? (Acc)vcol[q] : (Acc)0;
+  for (int q = 0; q < R; q++) acc[q] = (Acc)0;
+  if (!FOLD && acc_in && active) {
+#pragma unroll
+    for (int q = 0; q < R; q++)
+      if (q < nk) acc[q] = (Acc)vcol[q];
+  }
   const double x0 = g.ox + (double)i * g.dx, xn = g.ox + (double)(i + 1) * g.dx;
   const double y0 = g.oy + (double)j * g.dy, yn = g.oy + (double)(j + 1) * g.dy;
   // rows of the lane's slices that exist (one row per slice)
@@ -1151,17 +1162,32 @@ __device__ double par_bp_tile(const ParArgs &g, int tile, int zc, int a_begin, i
   if (!active) return 0.0;
   double ss = 0.0;
 #pragma unroll
-  for (int q = 0; q < R; q++)
-    if (q < nk) {
-      // slices without a row keep what they hold
-      float o;
-      if (FOLD && groups > 1)
-        o = (float)((Acc)vcol[q] + (q < nrow ? acc[q] : (Acc)0));
-      else
-        o = q < nrow ? (float)acc[q] : (!FOLD && acc_in ? vcol[q] : 0.0f);
-      vcol[q] = o;
-      ss += (double)o * (double)o;
+  for (int q4 = 0; q4 < R; q4 += 4) {
+    if (q4 + 4 <= nrow && !(FOLD && groups > 1)) {
+#pragma unroll
+      for (int q = q4; q < q4 + 4; q++) vcol[q] = (float)acc[q];
+      if (norm) {
+#pragma unroll
+        for (int q = q4; q < q4 + 4; q++) {
+          const float o = (float)acc[q];
+          ss += (double)o * (double)o;
+        }
+      }
+      continue;
     }
+#pragma unroll
+    for (int q = q4; q < q4 + 4; q++)
+      if (q < nk) {
+        // slices without a row keep what they hold
+        float o;
+        if (FOLD && groups > 1)
+          o = (float)((Acc)vcol[q] + (q < nrow ? acc[q] : (Acc)0));
+        else
+          o = q < nrow ? (float)acc[q] : (!FOLD && acc_in ? vcol[q] : 0.0f);
+        vcol[q] = o;
+        ss += (double)o * (double)o;
+      }
+  }
   return ss;
 }
 

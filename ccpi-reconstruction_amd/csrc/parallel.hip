@@ -109,8 +109,8 @@ __global__ __launch_bounds__(256) void par_bp_kernel(ParArgs g,
 // their partial sums to part[group] for par_bp_sum_kernel.  norm (one
 // group only): one partial of ||vol||^2 per workgroup.  5 waves per SIMD
 // (96 VGPRs, a few spills in the set-up): at 4 / 5 / 6 waves the
-// 512 x 512 x 32 BP takes 0.72 / 0.68 / 0.66 ms, 383 x 383 x 29 (ragged)
-// 0.31 / 0.24 / 0.24 and 256 x 256 x 16 0.065 / 0.066 / 0.068.  The
+// 512 x 512 x 32 BP takes 0.69 / 0.66 / 0.67 ms, 383 x 383 x 29 (ragged)
+// 0.29 / 0.23 / 0.24 and 256 x 256 x 16 0.059 / 0.061 / 0.064.  The
 // FP64-accumulation instances keep their registers.
 template <class Acc>
 constexpr int par_bp_lds_min_waves() { return std::is_same<Acc, float>::value ? 5 : 1; }
@@ -122,11 +122,14 @@ __attribute__((amdgpu_waves_per_eu(par_bp_lds_min_waves<Acc>(), 8))) void par_bp
     float *__restrict__ vol, float *__restrict__ part, int acc_in, double *__restrict__ norm) {
   extern __shared__ __align__(16) float smem[];
   const int grp = blockIdx.z;
-  const int a_begin = (int)((long long)g.na * grp / groups);
-  const int a_end = (int)((long long)g.na * (grp + 1) / groups);
+  // g.na * grp / groups in 32 bits
+  const int q = g.na / groups, rem = g.na % groups;
+  const int a_begin = q * grp + rem * grp / groups;
+  const int a_end = q * (grp + 1) + rem * (grp + 1) / groups;
   float *dst = groups == 1 ? vol : part + (size_t)grp * g.nx * g.ny * g.nz;
   const double ss = par_bp_tile<R, Acc>(g, blockIdx.x, blockIdx.y, a_begin, a_end, hmax, ab,
-                                        groups == 1 && acc_in != 0, sino, dst, smem);
+                                        groups == 1 && acc_in != 0, sino, dst, smem,
+                                        norm != nullptr);
   if (norm) block_part(ss, norm, (size_t)blockIdx.y * gridDim.x + blockIdx.x);
 }
 
