@@ -517,8 +517,8 @@ constexpr int kParShareWavesPerSimd = 7;
 constexpr int kParTileA = 32;
 
 // Workgroup `id` -> its rays and rows: ids go to the 8 XCDs in turn, each
-// XCD's in tiles of kParTileA angles of the same 64 columns; row blocks
-// slowest.  index: the workgroup's place among the live ones (ids past the
+// XCD's in tiles of kParTileA angles of the same 64 columns (par_tile_column);
+// row blocks slowest.  index: the workgroup's place among the live ones (ids past the
 // last tile are not live).
 struct ParShareItem {
   int a, h0, v0;
@@ -540,11 +540,12 @@ __device__ inline ParShareItem par_share_item(const ParArgs &g, int lr, int id) 
   const int rb = tile / (nb * nta), tab = tile - rb * (nb * nta);
   ParShareItem it;
   // uniform: the rays' and rows' addresses stay in scalar registers
-  it.a = __builtin_amdgcn_readfirstlane((tab / nb) * kParTileA + local % kParTileA);
-  it.h0 = __builtin_amdgcn_readfirstlane((tab % nb) * 64);
+  const int ta = tab / nb, c = par_tile_column(nb, ta, tab % nb);
+  it.a = __builtin_amdgcn_readfirstlane(ta * kParTileA + local % kParTileA);
+  it.h0 = __builtin_amdgcn_readfirstlane(c * 64);
   it.v0 = __builtin_amdgcn_readfirstlane(rb * 4 * lr);
   it.live = it.a < g.na && it.v0 < g.nv;
-  it.index = ((size_t)rb * g.na + it.a) * nb + tab % nb;
+  it.index = ((size_t)rb * g.na + it.a) * nb + c;
   return it;
 }
 

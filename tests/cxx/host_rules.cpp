@@ -62,6 +62,32 @@ static void cone_tiles() {
     }
 }
 
+// Every row of the parallel FP's tiles holds every column block once, and where
+// a block would keep to one or two XCDs and the middle half of the blocks
+// holds the work, no XCD has more than 1.5 times its share of it in 24 rows.
+static void par_columns() {
+  for (int nb = 1; nb <= 70; nb++) {
+    long long per[ccpi::kXcds] = {}, all = 0;
+    for (int ta = 0; ta < 24; ta++) {
+      std::vector<int> seen(nb);
+      for (int p = 0; p < nb; p++) {
+        const int c = ccpi::par_tile_column(nb, ta, p);
+        EXPECT(c >= 0 && c < nb);
+        if (c < 0 || c >= nb) return;
+        seen[c]++;
+        const bool middle = 4 * c >= nb - 1 && 4 * c <= 3 * nb - 1;
+        per[((long long)ta * nb + p) % ccpi::kXcds] += middle;
+        all += middle;
+      }
+      for (int s : seen) EXPECT(s == 1);
+    }
+    if (nb % 4 == 0)
+      for (long long p : per) EXPECT(2 * p * ccpi::kXcds <= 3 * all);
+  }
+  EXPECT(ccpi::par_tile_column(1 << 25, (1 << 26) + 3, (1 << 25) - 1) < 1 << 25);
+  EXPECT(ccpi::par_tile_column(1 << 25, (1 << 26) - 1, 0) >= 0);
+}
+
 // The tiled parallel BP's blocks leave room for five workgroups on a CU (160 KB,
 // handed out 1280 bytes at a time, with 128 bytes of the kernel's own) wherever
 // more than one angle is staged, and no angle less than fits is staged.
@@ -208,6 +234,7 @@ int main(int argc, char **argv) {
   const char *what = argc > 1 ? argv[1] : "";
   if (!std::strcmp(what, "grids")) grids();
   else if (!std::strcmp(what, "cone_tiles")) cone_tiles();
+  else if (!std::strcmp(what, "par_columns")) par_columns();
   else if (!std::strcmp(what, "bp_blocks")) bp_blocks();
   else if (!std::strcmp(what, "kept")) kept();
   else if (!std::strcmp(what, "kept_threads")) kept_threads();

@@ -19,7 +19,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("check", ["grids", "kept", "kept_threads", "refused_allocation",
-                                   "cone_tiles", "bp_blocks", "batch_tune"])
+                                   "cone_tiles", "par_columns", "bp_blocks", "batch_tune"])
 def test_host_rule(program, check):
     r = subprocess.run([program, check], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
