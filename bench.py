@@ -46,11 +46,11 @@ for p in (os.path.join(ROOT, "ccpi-reconstruction_amd"), os.path.join(ROOT, "ora
         sys.path.insert(0, p)
 
 HBM_PEAK_GBS = 8000.0
-KERNEL_SOURCES = ("cone.hip", "parallel.hip", "par_body.hpp", "common.hpp")
+KERNEL_SOURCES = ("cone.hip", "parallel.hip", "par_body.hpp", "common.hpp", "grid.hpp")
 # the sources each counter summary's kernels are built from
 SUMMARY_SOURCES = {
-    "cone512_projectors_counters.md": ("cone.hip", "common.hpp"),
-    "parallel_256x256x16_cgls.md": ("parallel.hip", "par_body.hpp", "common.hpp"),
+    "cone512_projectors_counters.md": ("cone.hip", "common.hpp", "grid.hpp"),
+    "parallel_256x256x16_cgls.md": ("parallel.hip", "par_body.hpp", "common.hpp", "grid.hpp"),
 }
 
 

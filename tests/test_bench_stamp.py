@@ -43,3 +43,13 @@ def test_summaries_stamp_known_sources():
         val, state = bench.measured_traffic(
             "cone_bp_kernel" if summary.startswith("cone") else "par_fp_kernel", summary)
         assert state in ("current", "stale") and (val is None) == (state == "stale")
+
+
+def test_stamps_cover_the_headers_of_their_sources():
+    import re
+    csrc = os.path.join(ROOT, "ccpi-reconstruction_amd", "csrc")
+    for names in [bench.KERNEL_SOURCES, *bench.SUMMARY_SOURCES.values()]:
+        for n in (n for n in names if n.endswith(".hpp")):
+            with open(os.path.join(csrc, n)) as f:
+                for h in re.findall(r'#include "(\w+\.hpp)"', f.read()):
+                    assert h in names, (n, h)
