@@ -913,7 +913,7 @@ __device__ inline double par_bp_thread(const ParArgs &g, int bx, int by, int tid
 // one coalesced copy per tile instead of each lane re-reading its columns'
 // rows, and with the columns' positions; every lane then weighs its own
 // column's footprint (the reference's FP64 arithmetic) on the staged rows.
-// Bound by vector issue (at 512 x 512 x 32 up to 87 % of the cycles, LDS 61 %,
+// Bound by vector issue (at 512 x 512 x 32 up to 89 % of the cycles, LDS 63 %,
 // half of it bank conflicts), 123 instructions per wavefront and angle of which
 // 64 are the 16 slices' products and sums.  So there are two blocks of LDS and the next one's reads go
 // straight there while this one is summed (one barrier a block, no register
